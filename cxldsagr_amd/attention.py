@@ -18,6 +18,7 @@ padding semantics and validation messages):
 Kernels: ``csrc/sparse_mla.hip`` and ``csrc/quantize.hip``.
 """
 
+import ctypes
 import math
 
 import torch
@@ -73,6 +74,15 @@ def _narrow_ids(indices, limit):
     return indices.contiguous()
 
 
+def _workspace(q, selected):
+    """The kernel's workspace for this call (None when it needs none), from
+    torch's allocator on the current stream, on which the kernels read it."""
+    needed = ctypes.c_int64()
+    _native.call("dsa_sparse_mla_workspace_bytes", q.shape[0], q.shape[1], selected,
+                 ctypes.byref(needed))
+    return torch.empty(needed.value, dtype=torch.uint8, device=q.device) if needed.value else None
+
+
 def sparse_mla(q, kv, indices, scale, value_dim=512):
     """Return BF16 ``[Q,H,512]`` sparse attention over bf16 ``kv [N,576]`` records.
 
@@ -90,13 +100,15 @@ def sparse_mla(q, kv, indices, scale, value_dim=512):
     q, kv = _aligned(q), _aligned(kv)
     ids = _narrow_ids(indices, kv.shape[0])
     with torch.cuda.device(q.device):
+        workspace = _workspace(q, ids.shape[1])
         _native.call(
-            "dsa_sparse_mla_bf16",
+            "dsa_sparse_mla_bf16_ws",
             _native.ptr(q), q.shape[0], q.shape[1],
             _native.ptr(kv), kv.shape[0],
             _native.ptr(ids), ids.shape[1],
             float(scale),
             _native.ptr(out),
+            _native.ptr(workspace), workspace.numel() if workspace is not None else 0,
             _native.stream_of(q.device),
         )
     return out
@@ -169,14 +181,16 @@ def sparse_mla_fp8_paged(q, kv_cache, page_table, indices, scale, value_dim=512,
     table = page_table.contiguous()
     ids = _narrow_ids(indices, n_tokens)
     with torch.cuda.device(q.device):
+        workspace = _workspace(q, ids.shape[1])
         _native.call(
-            "dsa_sparse_mla_fp8_paged",
+            "dsa_sparse_mla_fp8_paged_ws",
             _native.ptr(q), q.shape[0], q.shape[1],
             _native.ptr(cache), cache.shape[0],
             _native.ptr(table), n_tokens,
             _native.ptr(ids), ids.shape[1],
             float(scale),
             _native.ptr(out),
+            _native.ptr(workspace), workspace.numel() if workspace is not None else 0,
             _native.stream_of(q.device),
         )
     return out

@@ -691,16 +691,575 @@ __global__ __launch_bounds__(kThreads, 1) void sparse_mla_fwd(
   else run(std::false_type{});
 }
 
+// ---- few query rows: scores and values in two launches.
+//
+// (row, 64 heads) work-groups leave most CUs idle below 128 rows x 128 heads,
+// and a row's 64 key blocks are one serial chain of ~1.1 us steps. Splitting
+// the keys of one accumulation would make the fp32 sums depend on the batch
+// size; the work is split where it changes no sum, so the results have the
+// bits of sparse_mla_fwd:
+// * mla_scores: the scores of any key block are independent of the others.
+//   A work-group takes a row, 64 or 128 heads and a run of key blocks and
+//   writes the blocks' scores (fp32, -inf at padding) in the order of the PV
+//   operands, and each block's maximum per head.
+// * mla_values: the value dims are independent of each other. A work-group
+//   takes a row, 64 heads and 64 of the 512 dims, replays the running-max
+//   chain from the block maxima, forms P^T straight in the operand registers
+//   and runs the PV products block by block, in sparse_mla_fwd's order.
+// A block without a valid key changes no sum and is skipped.
+//
+// What bounds them at few rows: mla_scores (9 us for one row of 128 heads, 16
+// for 16) is a chain of load latencies, ids -> pages -> records -> LDS, in
+// front of one to four 1,152-cycle MFMA steps; from 64 rows on (34 us) the
+// 1 MB of fp32 scores per row it writes. mla_values (24 us for one row) is
+// one wave per SIMD issuing ~65 instructions per block (~650 cycles with the
+// LDS waits).
+constexpr int kScoreThreads = 512;
+constexpr int kScoreKeys = 1024;                      // most keys per work-group of mla_scores
+constexpr int kSplitSelected = 2048;                  // widest selection of the split form
+constexpr int kValueThreads = 256;
+constexpr int kValueBlocks = 2;                       // key blocks per step of mla_values
+constexpr int kValueKeys = kValueBlocks * kBlock;
+
+// 16 or 4 bytes of global memory at an address kept as an integer (a pointer
+// read back from LDS would be a generic one, whose loads count as LDS traffic
+// too and would be waited for at every barrier).
+template <typename T>
+__device__ __forceinline__ T global_read(uint64_t addr) {
+  return *(const T __attribute__((address_space(1)))*)addr;
+}
+
+// The records of positions first + tid + kThreadsN u (u < kBatch) of a
+// selection; the zero record for padding, an id outside [0, n_tokens) or a
+// page outside the cache. Ids, then pages, are loaded all at once.
+template <bool kFp8, int kThreadsN, int kBatch>
+__device__ __forceinline__ void resolve_records(const int32_t* __restrict__ ids, int first, int end,
+                                                const uint8_t* __restrict__ kv,
+                                                const int32_t* __restrict__ page_table,
+                                                int64_t n_tokens, int64_t pages,
+                                                uint64_t (&rec)[kBatch], bool (&valid)[kBatch]) {
+  int32_t id[kBatch], page[kBatch];
+#pragma unroll
+  for (int u = 0; u < kBatch; ++u) {
+    const int i = first + (int)threadIdx.x + kThreadsN * u;
+    id[u] = ids[i < end ? i : 0];
+    if (i >= end) id[u] = -1;
+  }
+#pragma unroll
+  for (int u = 0; u < kBatch; ++u) {
+    valid[u] = id[u] >= 0 && id[u] < n_tokens;
+    page[u] = kFp8 ? page_table[valid[u] ? id[u] / kPageTokens : 0] : 0;
+  }
+#pragma unroll
+  for (int u = 0; u < kBatch; ++u) {
+    valid[u] = valid[u] && (!kFp8 || (page[u] >= 0 && page[u] < pages));
+    const int64_t at = kFp8 ? (int64_t)page[u] * kPageTokens + id[u] % kPageTokens : (int64_t)id[u];
+    rec[u] = (uint64_t)(uintptr_t)(valid[u] ? kv + at * Format<kFp8>::kRecordBytes : zero_record);
+  }
+}
+
+// Scores of the split form: [row][block][head / 16][64 lanes][8] floats, lane
+// 16 g + c holding head c's key 2(j & 3) + 8(g & 1) + (g >> 1) + 16(j >> 2) at
+// j; block maxima (scaled): [row][block][head].
+constexpr int kScoreTile = 64 * 8;
+
+// Key blocks of a selection in the split form: whole rounds of mla_values
+// (blocks past the selection hold -inf scores).
+constexpr int kValueRound = 8;
+__host__ __device__ constexpr int padded_blocks(int64_t topk) {
+  return (int)((topk + kBlock * kValueRound - 1) / (kBlock * kValueRound)) * kValueRound;
+}
+
+// One work-group: kTiles head tiles of 32 (waves 0-3: tile wave % kTiles of
+// block wave / kTiles of the step), the K rows of a step's 4 / kTiles blocks
+// staged once as bf16 rows in LDS by waves 4-7, a step ahead.
+template <bool kFp8, int kTiles>
+__global__ __launch_bounds__(kScoreThreads, 1) void mla_scores(
+    const uint16_t* __restrict__ q, const uint8_t* __restrict__ kv,
+    const int32_t* __restrict__ page_table, int64_t n_tokens, int64_t pages,
+    const int32_t* __restrict__ indices, int64_t heads, int64_t topk, float scale_log2,
+    int32_t chunks, int32_t chunk_steps, float* __restrict__ scores,
+    float* __restrict__ block_max) {
+  using F = Format<kFp8>;
+  constexpr int kStepBlocks = 4 / kTiles;
+  constexpr int kStepKeys = kStepBlocks * kBlock;
+  // Staging: kLanes lanes per key, each 16-byte pieces of its record.
+  constexpr int kLanes = 256 / kStepKeys;
+  constexpr int kLatent = (kFp8 ? kVDim : 2 * kQkDim) / (16 * kLanes);
+  constexpr int kRope = kFp8 ? 8 / kLanes : 0;
+  // Register sets of records in flight: a step's records are loaded kDepth
+  // steps before they are staged.
+  constexpr int kDepth = kLatent + kRope > 10 ? 1 : kLatent + kRope > 6 ? 2 : 3;
+  __shared__ __align__(16) uint8_t rows_lds[2][kStepKeys * kRowBytes];
+  // This work-group's records (and the staging's look-ahead past them).
+  __shared__ uint64_t records[kScoreKeys + kDepth * kStepKeys];
+  __shared__ uint32_t valid_bits[kScoreKeys / 32];  // by block, bit = key
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const float neg_inf = -__builtin_inff();
+  const uint32_t groups = (uint32_t)(heads / (32 * kTiles));
+  const uint32_t chunk = blockIdx.x % (uint32_t)chunks;
+  const uint32_t rest = blockIdx.x / (uint32_t)chunks;
+  const int64_t head0 = (int64_t)(rest % groups) * (32 * kTiles);
+  const int64_t row = rest / groups;
+  const int n_blocks = padded_blocks(topk);
+  const int all_steps = n_blocks / kStepBlocks;
+  const int step0 = (int)chunk * chunk_steps;
+  const int steps = min(chunk_steps, all_steps - step0);
+  if (steps <= 0) return;
+  const int32_t* ids = indices + row * topk;
+  const int first = step0 * kStepKeys;
+
+  // The score waves' Q^T operands (k-step ks: dims 16 ks + 8h of head n), on
+  // their way while the records are looked up.
+  constexpr int kQOps = kQkDim / 16;
+  const int tile = wave % kTiles;
+  const int n = lane & 31;
+  const int h = lane >> 5;
+  v4u q_ops[kQOps];
+  if (wave < 4) {
+    const uint16_t* qrow = q + ((row * heads + head0 + 32 * tile + n) * kQkDim) + 8 * h;
+#pragma unroll
+    for (int ks = 0; ks < kQOps; ++ks) q_ops[ks] = *reinterpret_cast<const v4u*>(qrow + 16 * ks);
+  }
+  for (int i0 = 0; i0 < (steps + kDepth) * kStepKeys; i0 += kScoreThreads) {
+    uint64_t rec[1];
+    bool valid[1];
+    const int end = (int)(topk < first + steps * kStepKeys ? topk : first + steps * kStepKeys);
+    resolve_records<kFp8, kScoreThreads, 1>(ids, first + i0, end, kv, page_table, n_tokens, pages, rec, valid);
+    const int i = i0 + (int)threadIdx.x;
+    const uint64_t bits = __builtin_amdgcn_ballot_w64(valid[0]);
+    if (i < (steps + kDepth) * kStepKeys) records[i] = rec[0];
+    if (i < steps * kStepKeys && (lane & 31) == 0) valid_bits[i / 32] = (uint32_t)(bits >> (lane & 32));
+  }
+  __syncthreads();
+
+  if (wave < 4) {
+    // ---- score wave
+    const int blk = wave / kTiles;
+    constexpr int kQAgprs = 32;  // operands held in AGPRs (256 registers per wave, split 128 / 128)
+#pragma unroll
+    for (int ks = 0; ks < kQAgprs; ++ks) asm volatile("" : "+a"(q_ops[ks]));
+    const uint32_t k_lane = (uint32_t)(uintptr_t)&rows_lds[0][0] +
+                            (uint32_t)(blk * kBlock + score_key(n)) * kRowBytes + 16 * h;
+    // The scores of the previous step, finished (padding keys, maximum,
+    // stores) in slices under this step's MFMAs.
+    v16f prev = {};
+    uint32_t prev_mask = 0;
+    int prev_block = 0;
+    float mx = neg_inf;
+    auto finish = [&](int slice) __attribute__((always_inline)) {
+      if (slice < 8) {
+        mx = fmaxf(fmaxf(mx, prev[2 * slice]), prev[2 * slice + 1]);
+      } else if (slice == 8) {
+        const uint32_t ub = __float_as_uint(mx);
+        const auto sw32 = __builtin_amdgcn_permlane32_swap(ub, ub, false, false);
+        mx = fmaxf(__uint_as_float(sw32[0]), __uint_as_float(sw32[1])) * scale_log2;
+      } else if (slice < 13) {
+        const int ap = slice - 9;
+        float* dst = scores + (((row * n_blocks + prev_block) * (heads / 16)) + (head0 + 32 * tile) / 16 + (n >> 4)) * kScoreTile;
+        *reinterpret_cast<v4f*>(dst + ((2 * h + (ap & 1)) * 16 + (n & 15)) * 8 + 4 * (ap >> 1)) =
+            v4f{prev[4 * ap], prev[4 * ap + 1], prev[4 * ap + 2], prev[4 * ap + 3]};
+      } else if (slice == 13) {
+        if (h == 0) block_max[(row * n_blocks + prev_block) * heads + head0 + 32 * tile + n] = mx;
+      }
+    };
+    auto mask_padding = [&]() __attribute__((always_inline)) {
+      mx = neg_inf;
+      if (prev_mask != 0xFFFFFFFFu) {
+        // Key of register r: score_key(8 (r / 4) + 4 h + r % 4).
+        const uint32_t mine = prev_mask >> h;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) prev[r] = mine & (1u << score_key(8 * (r >> 2) + (r & 3))) ? prev[r] : neg_inf;
+      }
+    };
+    lds_barrier();  // step 0's rows
+    for (int t = 0; t < steps; ++t) {
+      const uint32_t kbase = k_lane + (uint32_t)(t & 1) * (uint32_t)sizeof(rows_lds[0]);
+      constexpr int kAheadK = 12;
+      v4u ka[kAheadK];
+#pragma unroll
+      for (int d = 0; d < kAheadK; ++d) ka[d] = lds_load<v4u>(kbase + 32 * d);
+      const uint32_t step_bits = valid_bits[t * kStepBlocks + blk];
+      v16f s = {};
+      if (t > 0) mask_padding();
+#pragma unroll
+      for (int ks = 0; ks < kQOps; ++ks) {
+        const v8bf a = as_v8bf(ka[ks % kAheadK]);
+        if (ks + kAheadK < kQOps) ka[ks % kAheadK] = lds_load<v4u>(kbase + 32 * (ks + kAheadK));
+        s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, as_v8bf(q_ops[ks]), s, 0, 0, 0);
+        if (ks >= 2 && ks < 11) finish(ks - 2);
+        if (ks == 11 && t > 0) {
+#pragma unroll
+          for (int i = 9; i < 14; ++i) finish(i);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      prev = s;
+      prev_mask = __builtin_amdgcn_readfirstlane(step_bits);
+      prev_block = (step0 + t) * kStepBlocks + blk;
+      lds_barrier();
+    }
+    mask_padding();
+#pragma unroll
+    for (int i = 0; i < 14; ++i) finish(i);
+    for (int t = steps; t % kDepth != 0; ++t) lds_barrier();  // the staging waves' whole rounds
+    return;
+  }
+
+  // ---- staging wave
+  const int slot = threadIdx.x - 256;
+  const int kk = slot / kLanes;
+  const int j = slot % kLanes;
+  v4u raw[kDepth][kLatent + kRope];
+  v4f tile_scales[kDepth] = {};
+  auto fetch = [&](int t, int set) __attribute__((always_inline)) {
+    const uint64_t rec = records[t * kStepKeys + kk];
+    const uint64_t mine = rec + 16 * j;
+#pragma unroll
+    for (int i = 0; i < kLatent; ++i) raw[set][i] = global_read<v4u>(mine + 16 * kLanes * i);
+#pragma unroll
+    for (int i = 0; i < kRope; ++i) raw[set][kLatent + i] = global_read<v4u>(mine + kVDim + 16 + 16 * kLanes * i);
+    if (kFp8) tile_scales[set] = global_read<v4f>(rec + kVDim);
+  };
+  auto stage = [&](int t, int set) __attribute__((always_inline)) {
+    const uint32_t at = (uint32_t)(uintptr_t)&rows_lds[0][0] + (uint32_t)(t & 1) * (uint32_t)sizeof(rows_lds[0]) +
+                        (uint32_t)kk * kRowBytes;
+#pragma unroll
+    for (int i = 0; i < kLatent; ++i) {
+      if (kFp8) {
+        const float sc = tile_scales[set][16 * kLanes * i / 128];
+        const v4u w = raw[set][i];
+        const uint32_t to = at + 32 * (uint32_t)(kLanes * i + j);
+        lds_store<v4u>(to, v4u{dequant_pair<false>(w.x, sc), dequant_pair<true>(w.x, sc),
+                               dequant_pair<false>(w.y, sc), dequant_pair<true>(w.y, sc)});
+        lds_store<v4u>(to + 16, v4u{dequant_pair<false>(w.z, sc), dequant_pair<true>(w.z, sc),
+                                    dequant_pair<false>(w.w, sc), dequant_pair<true>(w.w, sc)});
+      } else {
+        lds_store<v4u>(at + 16 * (uint32_t)(kLanes * i + j), raw[set][i]);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < kRope; ++i)
+      lds_store<v4u>(at + 2 * kVDim + 16 * (uint32_t)(kLanes * i + j), raw[set][kLatent + i]);
+  };
+#pragma unroll
+  for (int u = 0; u < kDepth; ++u) fetch(min(u, steps), u);
+  // Step t's rows are staged before the barrier that starts S(t); their
+  // buffer's last reader, S(t - 2), ended before the barrier before that one.
+  for (int t0 = 0; t0 < steps; t0 += kDepth) {
+#pragma unroll
+    for (int u = 0; u < kDepth; ++u) {
+      stage(t0 + u, u);  // past the last step: zero rows nobody reads
+      __builtin_amdgcn_sched_barrier(0);
+      fetch(min(t0 + u + kDepth, steps), u);
+      lds_barrier();
+    }
+  }
+  lds_barrier();  // the barrier after S(steps - 1)
+}
+
+// One work-group: a row, 64 heads (wave w: heads 16 w .. + 15) and kDv of the
+// value dims, in steps of kValueBlocks key blocks. Latency rules it (records,
+// scores and maxima come from the last-level cache or HBM), so all loads of a
+// step go out kDepth steps ahead.
+template <bool kFp8, int kDv, int kDepth>
+__global__ __launch_bounds__(kValueThreads, kDv < 256 ? 2 : 1) void mla_values(
+    const uint8_t* __restrict__ kv, const int32_t* __restrict__ page_table, int64_t n_tokens,
+    int64_t pages, const int32_t* __restrict__ indices, int64_t rows, int64_t heads, int64_t topk,
+    float scale_log2, const float* __restrict__ scores, const float* __restrict__ block_max,
+    uint16_t* __restrict__ out) {
+  // Value rows of a step, by parity: rows 4 or 36 (mod 64) dwords apart, so
+  // that the 8 even (or odd) keys of a V^T transpose read are on disjoint
+  // 8-bank windows.
+  constexpr int kStride = 2 * kDv + 16;
+  static_assert(kStride / 4 % 64 == 4 || kStride / 4 % 64 == 36, "bank windows of the transpose reads");
+  __shared__ __align__(16) uint8_t v_lds[2][kValueKeys * kStride];
+  __shared__ uint64_t records[kSplitSelected + (kDepth + 1) * kValueKeys];  // + the look-ahead
+  __shared__ int32_t wave_last[kValueThreads / 64];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c = lane & 15;
+  const int g = lane >> 4;
+  const float neg_inf = -__builtin_inff();
+  // Work-groups go to the XCDs round-robin by linear id: the parts of one
+  // (row, 64 heads), which read the same scores, are 8 ids apart and share an
+  // XCD's L2.
+  constexpr uint32_t kParts = kVDim / kDv;
+  const uint32_t groups = (uint32_t)(heads / 64);
+  const uint32_t tile = (blockIdx.x / (8 * kParts)) * 8 + (blockIdx.x & 7);
+  const int d0 = (int)((blockIdx.x >> 3) % kParts) * kDv;
+  const int64_t row = tile / groups;
+  if (row >= rows) return;
+  const int64_t head0 = (int64_t)(tile % groups) * 64 + 16 * wave;
+  const int32_t* ids = indices + row * topk;
+  const int n_blocks = padded_blocks(topk);
+
+  // Scores and maxima of this wave's 16 heads (uniform base, lane offset).
+  v4f s_lo[kDepth][kValueBlocks], s_hi[kDepth][kValueBlocks];
+  float mb[kDepth][kValueBlocks];
+  // (A row's scores are n_blocks x heads x 128 bytes: 32-bit offsets.)
+  const int64_t tiles16 = heads / 16;
+  const uint8_t* s_base = reinterpret_cast<const uint8_t*>(scores + (row * n_blocks * tiles16 + head0 / 16) * kScoreTile);
+  const uint8_t* m_base = reinterpret_cast<const uint8_t*>(block_max + row * n_blocks * heads + head0);
+  auto load_scores = [&](int t, int b, int set) __attribute__((always_inline)) {
+    // Past the last block: the last one again, not used.
+    const uint32_t block = (uint32_t)min(t * kValueBlocks + b, n_blocks - 1);
+    const uint32_t at = block * (uint32_t)(tiles16 * kScoreTile * 4) + 32u * (uint32_t)lane;
+    s_lo[set][b] = *reinterpret_cast<const v4f*>(s_base + at);
+    s_hi[set][b] = *reinterpret_cast<const v4f*>(s_base + at + 16);
+    mb[set][b] = *reinterpret_cast<const float*>(m_base + (block * (uint32_t)(heads * 4) + 4u * (uint32_t)c));
+  };
+
+  // Record rows of the whole selection, and the last valid position.
+  {
+    int32_t last = -1;
+    constexpr int kBatch = 8;
+    const int total = n_blocks * kBlock;
+    for (int i = threadIdx.x; i < (kDepth + 1) * kValueKeys; i += kValueThreads)
+      records[total + i] = (uint64_t)(uintptr_t)zero_record;
+    for (int i0 = 0; i0 < total; i0 += kBatch * kValueThreads) {
+      uint64_t rec[kBatch];
+      bool valid[kBatch];
+      resolve_records<kFp8, kValueThreads, kBatch>(ids, i0, (int)topk, kv, page_table, n_tokens, pages, rec, valid);
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u) {
+        const int i = i0 + (int)threadIdx.x + kValueThreads * u;
+        if (i < total) records[i] = rec[u] + (kFp8 ? d0 : 2 * d0);
+        if (valid[u]) last = i;
+      }
+    }
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) last = max(last, __shfl_xor(last, m));
+    if (lane == 0) wave_last[wave] = last;
+  }
+  __syncthreads();
+  const int last = __builtin_amdgcn_readfirstlane(
+      max(max(wave_last[0], wave_last[1]), max(wave_last[2], wave_last[3])));
+  static_assert(kValueRound % (kDepth * kValueBlocks) == 0, "whole rounds of the register sets");
+  // Steps up to the last valid position, in whole rounds of the register sets.
+  const int steps = (last + kDepth * kValueKeys) / (kDepth * kValueKeys) * kDepth;
+
+  // Staging: four lanes per key.
+  static_assert(4 * kValueKeys == kValueThreads, "a step's keys by four lanes each");
+  const int kk = threadIdx.x >> 2;
+  const int j = threadIdx.x & 3;
+  constexpr int kRaw = kDv / 64 * (kFp8 ? 1 : 2);
+  constexpr int kScales = kFp8 ? (kDv + 127) / 128 : 1;
+  v4u raw[kDepth][kRaw];
+  float tile_scale[kDepth][kScales] = {};
+  uint64_t rec_next = records[kk];  // of the next step to fetch
+  const int scale_at = kVDim + 4 * (d0 / 128) - d0;  // from the record's first value byte here
+  auto fetch = [&](int t, int set) __attribute__((always_inline)) {
+    const uint64_t rec = rec_next;
+    rec_next = records[(t + 1) * kValueKeys + kk];
+#pragma unroll
+    for (int u = 0; u < kRaw; ++u) raw[set][u] = global_read<v4u>(rec + 16 * j + 64 * u);
+    if (kFp8) {
+#pragma unroll
+      for (int u = 0; u < kScales; ++u) tile_scale[set][u] = global_read<float>(rec + scale_at + 4 * u);
+    }
+  };
+  const uint32_t v_base = (uint32_t)(uintptr_t)&v_lds[0][0];
+  auto stage = [&](int t, int set) __attribute__((always_inline)) {
+    const uint32_t to = v_base + (uint32_t)(t & 1) * (uint32_t)sizeof(v_lds[0]) + (uint32_t)kk * kStride;
+#pragma unroll
+    for (int u = 0; u < kRaw; ++u) {
+      const v4u w = raw[set][u];
+      if (kFp8) {
+        const float sc = tile_scale[set][u / 2];
+        lds_store<v4u>(to + 128 * u + 32 * j, v4u{dequant_pair<false>(w.x, sc), dequant_pair<true>(w.x, sc),
+                                                  dequant_pair<false>(w.y, sc), dequant_pair<true>(w.y, sc)});
+        lds_store<v4u>(to + 128 * u + 32 * j + 16, v4u{dequant_pair<false>(w.z, sc), dequant_pair<true>(w.z, sc),
+                                                       dequant_pair<false>(w.w, sc), dequant_pair<true>(w.w, sc)});
+      } else {
+        lds_store<v4u>(to + 64 * u + 16 * j, w);
+      }
+    }
+  };
+
+  constexpr int kM = kDv / 16;
+  v4f o[kM], l_acc = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int m = 0; m < kM; ++m) o[m] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+  float m_run = neg_inf;
+  const v8bf ones = as_v8bf(v4u{0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u});
+  const int vkey = 2 * (c >> 2) + 8 * (g & 1) + (g >> 1);
+  const uint32_t v_lane = v_base + (uint32_t)vkey * kStride + 8 * (c & 3);
+  // The running max of this lane's head through one block, as sparse_mla_fwd
+  // takes it, and the block's P^T operand; the rescale factor stays in alpha.
+  float alpha = 1.0f;
+  auto softmax = [&](float mx, const v4f& lo, const v4f& hi) __attribute__((always_inline)) -> v8bf {
+    const bool need = (mx > m_run + kRescaleThreshold) | ((m_run == neg_inf) & (mx != neg_inf));
+    const float m_new = need & (mx > m_run) ? mx : m_run;
+    alpha = need ? __builtin_amdgcn_exp2f(m_run - m_new) : 1.0f;
+    m_run = m_new;
+    const float neg_m = m_run == neg_inf ? 0.0f : -m_run;
+    auto p = [&](float v) { return __builtin_amdgcn_exp2f(__builtin_fmaf(v, scale_log2, neg_m)); };
+    return as_v8bf(v4u{pack_bf16(p(lo[0]), p(lo[1])), pack_bf16(p(lo[2]), p(lo[3])),
+                       pack_bf16(p(hi[0]), p(hi[1])), pack_bf16(p(hi[2]), p(hi[3]))});
+  };
+  if (steps > 0) {
+#pragma unroll
+    for (int u = 0; u < kDepth; ++u) {
+      fetch(u, u);
+#pragma unroll
+      for (int b = 0; b < kValueBlocks; ++b) load_scores(u, b, u);
+    }
+    // The softmax runs one block ahead of the PV products: its VALU work
+    // fills the LDS latency and the MFMAs of the block before.
+    v8bf p_next = softmax(mb[0][0], s_lo[0][0], s_hi[0][0]);
+    for (int t0 = 0; t0 < steps; t0 += kDepth) {
+#pragma unroll
+      for (int u = 0; u < kDepth; ++u) {
+        const int t = t0 + u;
+        stage(t, u);  // the buffer's last readers passed the previous barrier
+        __builtin_amdgcn_sched_barrier(0);
+        fetch(t + kDepth, u);
+        lds_barrier();
+        const uint32_t vb = v_lane + (uint32_t)(t & 1) * (uint32_t)sizeof(v_lds[0]);
+#pragma unroll
+        for (int b = 0; b < kValueBlocks; ++b) {
+          if (__builtin_amdgcn_ballot_w64(alpha != 1.0f)) {
+            l_acc *= alpha;
+#pragma unroll
+            for (int m = 0; m < kM; ++m) o[m] *= alpha;
+          }
+          const v8bf pb = p_next;
+          v4s v0[kM], v1[kM];
+#pragma unroll
+          for (int m = 0; m < kM; ++m) {
+            const uint32_t at = vb + (uint32_t)(b * kBlock) * kStride + 32 * m;
+            v0[m] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s)(uintptr_t)at);
+            v1[m] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s)(uintptr_t)(at + 16 * kStride));
+          }
+          // The next block's scores: in this step's set or the next one's.
+          const int nu = b + 1 < kValueBlocks ? u : (u + 1) % kDepth;
+          const int nb = b + 1 < kValueBlocks ? b + 1 : 0;
+          v4u p_regs = __builtin_bit_cast(v4u, softmax(mb[nu][nb], s_lo[nu][nb], s_hi[nu][nb]));
+          asm volatile("" : "+v"(p_regs));  // here, ahead of the MFMAs that wait for the V^T reads
+          p_next = as_v8bf(p_regs);
+          l_acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pb, l_acc, 0, 0, 0);
+#pragma unroll
+          for (int m = 0; m < kM; ++m) {
+            const v8bf va = __builtin_bit_cast(v8bf, __builtin_shufflevector(v0[m], v1[m], 0, 1, 2, 3, 4, 5, 6, 7));
+            o[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, pb, o[m], 0, 0, 0);
+          }
+        }
+        // Into the registers just read: loads into others would be copied
+        // here, and the copies would wait for them.
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int b = 0; b < kValueBlocks; ++b) load_scores(t + kDepth, b, u);
+      }
+    }
+  }
+
+  const float lt = l_acc[0];
+  const float inv_l = lt > 0.0f ? 1.0f / lt : 0.0f;
+  uint16_t* orow = out + ((row * heads + head0 + c) * kVDim) + d0 + 4 * g;
+#pragma unroll
+  for (int m = 0; m < kM; ++m)
+    *reinterpret_cast<uint2*>(orow + 16 * m) = make_uint2(pack_bf16(o[m][0] * inv_l, o[m][1] * inv_l),
+                                                          pack_bf16(o[m][2] * inv_l, o[m][3] * inv_l));
+}
+
+// How a call's rows are run: rows [0, wide_rows) by sparse_mla_fwd, the rest in
+// the split form with kDv = dv.
+//
+// sparse_mla_fwd takes about 78 us (2,048 selected) for each round of one
+// (row, 64 heads) work-group per CU, however few there are. The split form,
+// whose scores go through memory instead of LDS, measured 35 / 43 / 54 / 77 us
+// for 4 / 16 / 32 / 64 rows of 128 heads over 2,048 fp8 records (56 / 92 us
+// for 32 / 64 rows of bf16 records), so the rows after the last full round go
+// there while they are at most a quarter of a round. It also wants some
+// length to spread: at 500 selected 19.7 us against 26.4, at 33 20.0 against
+// 17.6.
+struct MlaPlan {
+  int64_t wide_rows, split_rows;
+  int dv;
+  int64_t score_floats, bytes;  // of the split rows' workspace: scores, then block maxima
+};
+
+constexpr int64_t kSplitMinSelected = 320;
+
+MlaPlan mla_plan(int64_t rows, int64_t heads, int64_t topk) {
+  MlaPlan p{rows, 0, 0, 0, 0};
+  const int64_t cus = device_cu_count();
+  const int64_t per_row = heads / kHeadsPerGroup;
+  if (topk < kSplitMinSelected || topk > kSplitSelected || per_row * 4 > cus) return p;
+  const int64_t round = cus / per_row;  // rows of a full round
+  const int64_t tail = rows % round;
+  if (tail == 0 || tail * per_row * 4 > cus) return p;
+  p.wide_rows = rows - tail;
+  p.split_rows = tail;
+  // One round of mla_values work-groups at 64 dims up to an eighth of the
+  // CUs' tiles; above, 128 dims halve the softmax work (each part of the
+  // dims repeats it).
+  p.dv = tail * per_row * 8 <= cus ? 64 : 128;
+  p.score_floats = tail * padded_blocks(topk) * heads * kBlock;
+  p.bytes = (p.score_floats + tail * padded_blocks(topk) * heads) * 4;
+  return p;
+}
+
 template <bool kFp8>
-int launch(const void* q, int64_t rows, int64_t heads, const void* kv, const int32_t* page_table,
+int launch_split(const MlaPlan& p, const uint16_t* q, int64_t heads, const uint8_t* kv,
+                 const int32_t* page_table, int64_t n_tokens, int64_t pages, const int32_t* indices,
+                 int64_t topk, float scale_log2, uint16_t* out, float* scores, hipStream_t stream) {
+  const int64_t rows = p.split_rows;
+  float* block_max = scores + p.score_floats;
+  // mla_scores: all heads of a multiple of 128 share a staged block, and the
+  // blocks are dealt out for about one work-group per CU.
+  const int tiles = heads % 128 == 0 ? 4 : 2;
+  const int64_t steps = padded_blocks(topk) * tiles / 4;
+  const int64_t units = rows * (heads / (32 * tiles));
+  const int64_t most = kScoreKeys / kBlock * tiles / 4;
+  int64_t chunk = (units * steps + device_cu_count() - 1) / device_cu_count();
+  if (chunk > most) chunk = most;
+  const int64_t chunks = (steps + chunk - 1) / chunk;
+  hipLaunchKernelGGL((tiles == 4 ? mla_scores<kFp8, 4> : mla_scores<kFp8, 2>),
+                     dim3((unsigned)(units * chunks)), dim3(kScoreThreads), 0, stream, q, kv,
+                     page_table, n_tokens, pages, indices, heads, topk, scale_log2,
+                     (int32_t)chunks, (int32_t)chunk, scores, block_max);
+  DSA_CHECK_LAUNCH("sparse MLA scores");
+  const int64_t groups = (rows * (heads / 64) + 7) / 8;
+  hipLaunchKernelGGL((p.dv == 64 ? mla_values<kFp8, 64, 4> : mla_values<kFp8, 128, 4>),
+                     dim3((unsigned)(groups * 8 * (kVDim / p.dv))), dim3(kValueThreads), 0, stream,
+                     kv, page_table, n_tokens, pages, indices, rows, heads, topk, scale_log2,
+                     scores, block_max, out);
+  DSA_CHECK_LAUNCH("sparse MLA values");
+  return kOk;
+}
+
+template <bool kFp8>
+int launch(const void* q_, int64_t rows, int64_t heads, const void* kv_, const int32_t* page_table,
            int64_t n_tokens, int64_t pages, const int32_t* indices, int64_t topk, float scale,
-           void* out, hipStream_t stream) {
+           void* out_, void* workspace, int64_t workspace_bytes, hipStream_t stream) {
+  const uint16_t* q = static_cast<const uint16_t*>(q_);
+  const uint8_t* kv = static_cast<const uint8_t*>(kv_);
+  uint16_t* out = static_cast<uint16_t*>(out_);
   const float scale_log2 = scale * 1.4426950408889634f;
-  hipLaunchKernelGGL(sparse_mla_fwd<kFp8>, dim3((unsigned)rows, (unsigned)(heads / kHeadsPerGroup)),
-                     dim3(kThreads), 0, stream, static_cast<const uint16_t*>(q),
-                     static_cast<const uint8_t*>(kv), page_table, n_tokens, pages, indices, heads,
-                     topk, scale_log2, static_cast<uint16_t*>(out));
-  DSA_CHECK_LAUNCH("sparse MLA");
+  MlaPlan p = mla_plan(rows, heads, topk);
+  // The running max is taken on raw scores times scale_log2: an empty
+  // block's -inf stays -inf (and the split form may skip it) only for
+  // positive scales.
+  if (workspace == nullptr || !(scale_log2 > 0.0f)) p = MlaPlan{rows, 0, 0, 0, 0};
+  if (p.split_rows > 0) {
+    DSA_CHECK_ARG(reinterpret_cast<uintptr_t>(workspace) % 16 == 0 && workspace_bytes >= p.bytes,
+                  "sparse MLA workspace too small or misaligned");
+  }
+  if (p.wide_rows > 0) {
+    hipLaunchKernelGGL(sparse_mla_fwd<kFp8>,
+                       dim3((unsigned)p.wide_rows, (unsigned)(heads / kHeadsPerGroup)),
+                       dim3(kThreads), 0, stream, q, kv, page_table, n_tokens, pages, indices,
+                       heads, topk, scale_log2, out);
+    DSA_CHECK_LAUNCH("sparse MLA");
+  }
+  if (p.split_rows > 0)
+    return launch_split<kFp8>(p, q + p.wide_rows * heads * kQkDim, heads, kv, page_table, n_tokens,
+                              pages, indices + p.wide_rows * topk, topk, scale_log2,
+                              out + p.wide_rows * heads * kVDim, static_cast<float*>(workspace),
+                              stream);
   return kOk;
 }
 
@@ -722,9 +1281,21 @@ int check_common(const void* q, int64_t rows, int64_t heads, const int32_t* indi
 }  // namespace
 }  // namespace dsa
 
-extern "C" int dsa_sparse_mla_bf16(const void* q, int64_t rows, int64_t heads, const void* kv,
-                                   int64_t kv_rows, const int32_t* indices, int64_t topk,
-                                   float scale, void* out, hipStream_t stream) {
+extern "C" int dsa_sparse_mla_workspace_bytes(int64_t rows, int64_t heads, int64_t topk,
+                                              int64_t* bytes) {
+  using namespace dsa;
+  DSA_CHECK_ARG(bytes != nullptr, "null pointer");
+  // (Shapes the operators refuse need none.)
+  *bytes = 0;
+  if (rows <= 0 || rows >= 0x7FFFFFFF || heads <= 0 || heads % kHeadsPerGroup) return kOk;
+  *bytes = mla_plan(rows, heads, topk).bytes;
+  return kOk;
+}
+
+extern "C" int dsa_sparse_mla_bf16_ws(const void* q, int64_t rows, int64_t heads, const void* kv,
+                                      int64_t kv_rows, const int32_t* indices, int64_t topk,
+                                      float scale, void* out, void* workspace,
+                                      int64_t workspace_bytes, hipStream_t stream) {
   using namespace dsa;
   int status = check_common(q, rows, heads, indices, topk, scale, out);
   if (status != kOk || rows == 0) return status;
@@ -732,14 +1303,22 @@ extern "C" int dsa_sparse_mla_bf16(const void* q, int64_t rows, int64_t heads, c
   DSA_CHECK_ARG(kv != nullptr, "null kv");
   DSA_CHECK_ARG(reinterpret_cast<uintptr_t>(kv) % 16 == 0, "kv must be 16-byte aligned");
   return launch<false>(q, rows, heads, kv, nullptr, kv_rows, 0, indices, topk, scale, out,
-                       stream);
+                       workspace, workspace_bytes, stream);
 }
 
-extern "C" int dsa_sparse_mla_fp8_paged(const void* q, int64_t rows, int64_t heads,
-                                        const void* cache, int64_t pages,
-                                        const int32_t* page_table, int64_t n_tokens,
-                                        const int32_t* indices, int64_t topk, float scale,
-                                        void* out, hipStream_t stream) {
+extern "C" int dsa_sparse_mla_bf16(const void* q, int64_t rows, int64_t heads, const void* kv,
+                                   int64_t kv_rows, const int32_t* indices, int64_t topk,
+                                   float scale, void* out, hipStream_t stream) {
+  return dsa_sparse_mla_bf16_ws(q, rows, heads, kv, kv_rows, indices, topk, scale, out, nullptr, 0,
+                                stream);
+}
+
+extern "C" int dsa_sparse_mla_fp8_paged_ws(const void* q, int64_t rows, int64_t heads,
+                                           const void* cache, int64_t pages,
+                                           const int32_t* page_table, int64_t n_tokens,
+                                           const int32_t* indices, int64_t topk, float scale,
+                                           void* out, void* workspace, int64_t workspace_bytes,
+                                           hipStream_t stream) {
   using namespace dsa;
   int status = check_common(q, rows, heads, indices, topk, scale, out);
   if (status != kOk || rows == 0) return status;
@@ -749,5 +1328,14 @@ extern "C" int dsa_sparse_mla_fp8_paged(const void* q, int64_t rows, int64_t hea
   DSA_CHECK_ARG(cache && page_table, "null cache or page table");
   DSA_CHECK_ARG(reinterpret_cast<uintptr_t>(cache) % 16 == 0, "cache must be 16-byte aligned");
   return launch<true>(q, rows, heads, cache, page_table, n_tokens, pages, indices, topk, scale,
-                      out, stream);
+                      out, workspace, workspace_bytes, stream);
+}
+
+extern "C" int dsa_sparse_mla_fp8_paged(const void* q, int64_t rows, int64_t heads,
+                                        const void* cache, int64_t pages,
+                                        const int32_t* page_table, int64_t n_tokens,
+                                        const int32_t* indices, int64_t topk, float scale,
+                                        void* out, hipStream_t stream) {
+  return dsa_sparse_mla_fp8_paged_ws(q, rows, heads, cache, pages, page_table, n_tokens, indices,
+                                     topk, scale, out, nullptr, 0, stream);
 }

@@ -408,6 +408,25 @@ int dsa_sparse_mla_fp8_paged(const void* q, int64_t rows, int64_t heads, const v
                              hipStream_t stream);
 
 /*
+ * The same two operators with a workspace for their split form, which runs
+ * the rows after the last full round of work-groups (few rows: all of them)
+ * as block scores and value products in two launches. The results have the
+ * same bits with and without it. `workspace` is 16-byte aligned and holds at
+ * least dsa_sparse_mla_workspace_bytes (0: the split form is not used) bytes,
+ * needs no initialisation, and is free again when the stream has passed the
+ * call; null = no split form.
+ */
+int dsa_sparse_mla_workspace_bytes(int64_t rows, int64_t heads, int64_t topk, int64_t* bytes);
+int dsa_sparse_mla_bf16_ws(const void* q, int64_t rows, int64_t heads, const void* kv,
+                           int64_t kv_rows, const int32_t* indices, int64_t topk, float scale,
+                           void* out, void* workspace, int64_t workspace_bytes,
+                           hipStream_t stream);
+int dsa_sparse_mla_fp8_paged_ws(const void* q, int64_t rows, int64_t heads, const void* cache,
+                                int64_t pages, const int32_t* page_table, int64_t n_tokens,
+                                const int32_t* indices, int64_t topk, float scale, void* out,
+                                void* workspace, int64_t workspace_bytes, hipStream_t stream);
+
+/*
  * A11 - gather whole records from pinned host memory into device memory,
  * device[device_ids[r]] = host[host_ids[r]] for r < count, or for
  * r < *valid_count when valid_count (a device int64 or uint32 scalar, kind

@@ -1,0 +1,83 @@
+"""The split form of sparse MLA (scores and values in two launches, taken for
+the rows after the last full round of work-groups) gives the bits of the
+one-launch kernel, which the C entries without a workspace run."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+SCALE = 576**-0.5
+
+
+def _one_launch(q, cache, table, kv, ids, n_tokens, scale):
+    from cxldsagr_amd import _native
+
+    out = torch.empty(*q.shape[:2], 512, dtype=q.dtype, device=q.device)
+    if kv is None:
+        _native.call("dsa_sparse_mla_fp8_paged", _native.ptr(q), q.shape[0], q.shape[1],
+                     _native.ptr(cache), cache.shape[0], _native.ptr(table), n_tokens,
+                     _native.ptr(ids), ids.shape[1], scale, _native.ptr(out),
+                     _native.stream_of(q.device))
+    else:
+        _native.call("dsa_sparse_mla_bf16", _native.ptr(q), q.shape[0], q.shape[1],
+                     _native.ptr(kv), kv.shape[0], _native.ptr(ids), ids.shape[1], scale,
+                     _native.ptr(out), _native.stream_of(q.device))
+    return out
+
+
+# Rows around the bounds of the rule (an eighth and a quarter of a round of 256
+# work-groups, one row past a full round), selections around its shortest and
+# longest, off the 32-key block, the 64-key step and the 256-key round.
+@pytest.mark.parametrize("rows,heads,selected", [
+    (1, 128, 2048), (1, 64, 321), (2, 192, 1000), (16, 128, 2047), (17, 128, 545),
+    (32, 128, 2048), (33, 128, 700), (64, 64, 1025), (65, 64, 320), (129, 128, 640),
+    (160, 128, 351), (161, 128, 352), (3, 128, 319), (3, 128, 2049), (5, 64, 511),
+])
+def test_split_form_has_the_bits_of_one_launch(gpu, rows, heads, selected):
+    from cxldsagr_amd.attention import pack_kv_fp8, sparse_mla, sparse_mla_fp8_paged
+
+    gen = torch.Generator(device=gpu).manual_seed(rows * 4096 + selected)
+    tokens = 5000
+    pages = (tokens + 63) // 64
+    kv = torch.randn(tokens, 576, generator=gen, device=gpu).bfloat16()
+    table = torch.randperm(pages, generator=gen, device=gpu).int()
+    cache = torch.zeros(pages, 64, 656, dtype=torch.uint8, device=gpu)
+    pack_kv_fp8(kv, cache, table)
+    q = torch.randn(rows, heads, 576, generator=gen, device=gpu).bfloat16()
+    q[-1] *= 16  # peaked scores: the running max rises block after block
+    ids = torch.randint(0, tokens, (rows, selected), generator=gen, device=gpu).int()
+    # Padding: tails of every length in the last rows, holes and whole blocks,
+    # an empty row, a row of out-of-range ids, an infinite record.
+    keep = torch.randint(0, selected + 1, (rows, 1), generator=gen, device=gpu)
+    tail = torch.arange(selected, device=gpu) >= keep
+    ids[1::3] = torch.where(tail, -1, ids)[1::3]
+    ids[0, 32:128] = -1
+    ids[0, ::7] = -1
+    if rows > 2:
+        ids[1] = -1
+        ids[2] = tokens + 5
+    if rows > 3:
+        kv[7, 100] = float("inf")
+        ids[3, selected // 2] = 7
+    paged = sparse_mla_fp8_paged(q, cache, table, ids, SCALE, n_tokens=tokens)
+    flat = sparse_mla(q, kv, ids, SCALE)
+    for got, records in ((paged, None), (flat, kv)):
+        want = _one_launch(q, cache, table, records, ids, tokens, SCALE)
+        torch.cuda.synchronize()
+        same = (got.view(torch.int16) == want.view(torch.int16)) | (got.isnan() & want.isnan())
+        assert bool(same.all())
+
+
+def test_negative_and_zero_scales_take_one_launch(gpu):
+    """The split form skips a block by its -inf maximum, which holds for
+    positive scales only; others run as without a workspace."""
+    from cxldsagr_amd.attention import sparse_mla
+
+    gen = torch.Generator(device=gpu).manual_seed(3)
+    kv = torch.randn(900, 576, generator=gen, device=gpu).bfloat16()
+    q = torch.randn(4, 64, 576, generator=gen, device=gpu).bfloat16()
+    ids = torch.randint(0, 900, (4, 640), generator=gen, device=gpu).int()
+    for scale in (-SCALE, 0.0):
+        want = _one_launch(q, None, None, kv, ids, 0, scale)
+        assert torch.equal(sparse_mla(q, kv, ids, scale).view(torch.int16), want.view(torch.int16))
