@@ -81,3 +81,27 @@ def test_negative_and_zero_scales_take_one_launch(gpu):
     for scale in (-SCALE, 0.0):
         want = _one_launch(q, None, None, kv, ids, 0, scale)
         assert torch.equal(sparse_mla(q, kv, ids, scale).view(torch.int16), want.view(torch.int16))
+
+
+@pytest.mark.parametrize("heads", [64, 192])
+def test_rows_that_end_in_padding_equal_their_short_selections(gpu, heads):
+    """Rows stop at their last id in range: a full round of rows whose ids end
+    at every edge of the 64-key step has, row by row, the bits of the same ids
+    without the padding (a page table shorter than the ids' range and ids past
+    the cache count as padding)."""
+    from cxldsagr_amd.attention import sparse_mla
+
+    gen = torch.Generator(device=gpu).manual_seed(11)
+    rows, selected, tokens = 256 if heads == 64 else 85, 300, 1000
+    kv = torch.randn(tokens, 576, generator=gen, device=gpu).bfloat16()
+    q = torch.randn(rows, heads, 576, generator=gen, device=gpu).bfloat16()
+    ids = torch.randint(0, tokens, (rows, selected), generator=gen, device=gpu).int()
+    ends = [0, 1, 31, 32, 33, 63, 64, 65, 127, 128, 129, 191, 192, 255, 256, 257, 299, 300]
+    for r in range(rows):
+        ids[r, ends[r % len(ends)]:] = -1 if r % 2 else tokens
+    got = sparse_mla(q, kv, ids, SCALE)
+    for r in range(len(ends)):
+        end = ends[r]
+        want = (sparse_mla(q[r:r + 1], kv, ids[r:r + 1, :end].contiguous(), SCALE)[0] if end
+                else torch.zeros_like(got[r]))
+        assert torch.equal(got[r].view(torch.int16), want.view(torch.int16)), end
