@@ -161,7 +161,7 @@ __global__ __launch_bounds__(kThreads, 1) void sparse_mla_fwd(
   using F = Format<kFp8>;
   __shared__ Lds lds;
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 4;
   const int c = lane & 15;
   // Work-groups go to the XCDs round-robin by linear id: the head groups of a
