@@ -160,7 +160,7 @@ __global__ __launch_bounds__(kThreads, 1) void logits_fp8_mfma(
     const float* __restrict__ kscale, const int32_t* __restrict__ starts,
     const int32_t* __restrict__ ends, int64_t query_start, int64_t rows, int64_t columns,
     int64_t ldo, int64_t keys_per_split, const float* __restrict__ q_fold, float* __restrict__ out,
-    uint32_t* __restrict__ digit_counts, EmitArgs emit) {
+    uint32_t* __restrict__ digit_counts, EmitArgs emit, uint32_t qgroups) {
   constexpr bool kCount = kMode == kModeCount;
   constexpr bool kEmit = kMode == kModeEmit;
   __shared__ __align__(16) uint8_t ring[kRing][kStageBytes];
@@ -178,9 +178,15 @@ __global__ __launch_bounds__(kThreads, 1) void logits_fp8_mfma(
   const int lane = tid & 63;
   const int group = lane >> 4;
   const int col = lane & 15;
-  const int64_t q0 = (int64_t)blockIdx.y * kQueriesPerBlock;
-  const int64_t kb = (int64_t)blockIdx.x * keys_per_split;
-  if (kb >= ldo) return;  // a padding split (whole work-group, before any barrier)
+  // Work-groups go to the XCDs round-robin by linear id: XCD e takes the e-th
+  // eighth of the (key split, query group) pairs in split order, so each XCD
+  // gets as many pairs as the others and the query groups of a key range
+  // share its keys through one XCD's L2.
+  const uint32_t pair = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  const uint32_t split = pair / qgroups;
+  const int64_t q0 = (int64_t)(pair % qgroups) * kQueriesPerBlock;
+  const int64_t kb = (int64_t)split * keys_per_split;
+  if (kb >= ldo) return;  // past the last pair (whole work-group, before any barrier)
   const int64_t ke = kb + keys_per_split < ldo ? kb + keys_per_split : ldo;
   const float neg_inf = -__builtin_inff();
   // Keys of this split that the digit counts cover.
@@ -339,7 +345,7 @@ __global__ __launch_bounds__(kThreads, 1) void logits_fp8_mfma(
     }
   }
   auto list_of = [&](int64_t row) {
-    return emit.lists + (row * emit.splits + blockIdx.x) * (int64_t)emit.cap;
+    return emit.lists + (row * emit.splits + split) * (int64_t)emit.cap;
   };
 
   // Wave 0's finished rows, [stage parity][query][key].
@@ -543,13 +549,13 @@ __global__ __launch_bounds__(kThreads, 1) void logits_fp8_mfma(
     if (wave != 0 && lane < kQueriesPerWave) {
       const int64_t row = qw + lane;
       if (row < rows) {
-        uint32_t* rec = emit.records + (row * emit.splits + blockIdx.x) * 2;
+        uint32_t* rec = emit.records + (row * emit.splits + split) * 2;
         rec[0] = (uint32_t)(lane == 0 ? listed[0] : listed[1]);
         rec[1] = (uint32_t)(lane == 0 ? spill[0] : spill[1]);
       }
     }
     if (wave == w0_writer && lane < kQueriesPerWave && q0 + lane < rows) {
-      uint32_t* rec = emit.records + ((q0 + lane) * emit.splits + blockIdx.x) * 2;
+      uint32_t* rec = emit.records + ((q0 + lane) * emit.splits + split) * 2;
       rec[0] = (uint32_t)w0_state[lane][0];
       rec[1] = (uint32_t)w0_state[lane][1];
     }
@@ -674,28 +680,43 @@ __global__ __launch_bounds__(kFloorThreads) void index_floors(
 namespace dsa {
 namespace {
 
-// Key range per work-group: the grid is about one work-group per CU.
+// Key range per work-group. `splits` is the stride of the per-split output
+// (a multiple of 8 from 8 on); `live` of them hold keys and are launched, for
+// each query group.
 struct SplitPlan {
-  int64_t qgroups, splits, per;
+  int64_t qgroups, splits, per, live;
+  unsigned grid() const { return (unsigned)((live * qgroups + 7) / 8 * 8); }
 };
+
+// The split with the least time by rounds of one work-group per CU, each
+// kStartUs (operands and first keys) plus kStageUs per 128 keys (the stage's
+// MFMAs; both measured). Splitting for at least one work-group per CU and
+// padding the splits to a multiple of 8 left a few work-groups, or one XCD's,
+// to a second round that took as long as the first: 100 rows x 50,001 keys
+// 81.8 -> 48.0 us, 200 rows x 16,584 keys 59.8 -> 34.6 us.
+constexpr double kStartUs = 8.0, kStageUs = 3.0;
 
 SplitPlan split_plan(int64_t rows, int64_t ldo, bool counted) {
   SplitPlan p;
   p.qgroups = (rows + kQueriesPerBlock - 1) / kQueriesPerBlock;
   const int64_t cus = device_cu_count();
-  int64_t splits = (cus + p.qgroups - 1) / p.qgroups;
-  if (splits < 1) splits = 1;
-  int64_t per = (ldo + splits - 1) / splits;
-  per = (per + kStageKeys - 1) / kStageKeys * kStageKeys;
-  if (counted && per > kMaxSplitKeys) per = kMaxSplitKeys;  // 16-bit LDS counters
-  splits = (ldo + per - 1) / per;
-  // Work-groups are dealt to the eight XCDs round-robin by linear id
-  // (x + splits * y): with a multiple of 8 splits every query group of one
-  // key range runs on the same XCD and the eight share its keys through that
-  // XCD's L2. The added splits start past the last column and exit at once.
-  if (splits >= 8) splits = (splits + 7) / 8 * 8;
-  p.splits = splits;
-  p.per = per;
+  const int64_t stages = (ldo + kStageKeys - 1) / kStageKeys;
+  const int64_t most = stages < cus ? stages : cus;
+  double best = 0.0;
+  p.per = stages * kStageKeys;
+  for (int64_t s = 1; s <= most; ++s) {
+    const int64_t per_stages = (stages + s - 1) / s;
+    const int64_t live = (stages + per_stages - 1) / per_stages;
+    const int64_t rounds = (live * p.qgroups + cus - 1) / cus;
+    const double cost = (double)rounds * (kStartUs + kStageUs * (double)per_stages);
+    if (s == 1 || cost < best) {
+      best = cost;
+      p.per = per_stages * kStageKeys;
+    }
+  }
+  if (counted && p.per > kMaxSplitKeys) p.per = kMaxSplitKeys;  // 16-bit LDS counters
+  p.live = (ldo + p.per - 1) / p.per;
+  p.splits = p.live >= 8 ? (p.live + 7) / 8 * 8 : p.live;
   return p;
 }
 
@@ -732,10 +753,10 @@ int logits_launch(const void* q, const void* k, const float* weights, const floa
   DSA_CHECK_ARG(out != nullptr, "null pointer");
   const SplitPlan p = split_plan(rows, ldo, digit_counts != nullptr);
   hipLaunchKernelGGL(digit_counts ? logits_fp8_mfma<kModeCount> : logits_fp8_mfma<kModePlain>,
-                     dim3((unsigned)p.splits, (unsigned)p.qgroups), dim3(kThreads), 0, stream,
+                     dim3(p.grid()), dim3(kThreads), 0, stream,
                      static_cast<const uint8_t*>(q), static_cast<const uint8_t*>(k), weights,
                      kscale, starts, ends, query_start, rows, columns, ldo, p.per, q_fold, out,
-                     digit_counts, EmitArgs{});
+                     digit_counts, EmitArgs{}, (uint32_t)p.qgroups);
   DSA_CHECK_LAUNCH("indexer logits");
   return kOk;
 }
@@ -889,10 +910,11 @@ extern "C" int dsa_indexer_logits_fp8_emit(const void* q, const void* k, const f
                 reinterpret_cast<uint64_t*>(base + l.lists_offset),
                 reinterpret_cast<uint32_t*>(base + l.records_offset), (int32_t)l.cap,
                 (int32_t)l.plan.splits};
-  hipLaunchKernelGGL(logits_fp8_mfma<kModeEmit>, dim3((unsigned)l.plan.splits, (unsigned)l.plan.qgroups),
+  hipLaunchKernelGGL(logits_fp8_mfma<kModeEmit>, dim3(l.plan.grid()),
                      dim3(kThreads), 0, stream, static_cast<const uint8_t*>(q),
                      static_cast<const uint8_t*>(k), weights, kscale, starts, ends, query_start,
-                     rows, columns, ldo, l.plan.per, q_fold, scores, nullptr, emit);
+                     rows, columns, ldo, l.plan.per, q_fold, scores, nullptr, emit,
+                     (uint32_t)l.plan.qgroups);
   DSA_CHECK_LAUNCH("indexer logits (candidates)");
   return kOk;
 }
