@@ -778,8 +778,12 @@ EmitLayout emit_layout(int64_t rows, int64_t columns, int64_t list_cap) {
   const int64_t ldo = (columns + 255) / 256 * 256;
   l.plan = split_plan(rows, ldo, false);
   // Default: an eighth of the split (~2x the expected candidates of a split
-  // at a uniform spread).
+  // at a uniform spread of 64K columns), and at least 256 or the whole split:
+  // the rows of few and short splits list a larger share of them, and a list
+  // spills once fewer than 64 slots are left (with 64 in all, after its first
+  // candidate).
   int64_t cap = list_cap > 0 ? list_cap : l.plan.per / 8;
+  if (list_cap <= 0 && cap < 256) cap = l.plan.per < 256 ? l.plan.per : 256;
   cap = (cap + 63) / 64 * 64;
   if (cap < 64) cap = 64;
   l.cap = cap;

@@ -1158,32 +1158,21 @@ union FinishShared {
   FinishSort fs;
 };
 
-// One counting sort of the n candidate keys (unique composite keys whose
-// radix keys lie in [lo, hi]) held kSortPerThread per thread (slot j of a
-// thread holds a key when bit j of `valid` is set): kSortBins linear
-// buckets of the radix keys,
-// ranks inside a bucket by comparison, the first `count` through LDS to
-// emit(i, key). Buckets that start at or past `count` hold no output key and
-// are neither ranked nor limited in size. fs.cursor and fs.crowded must be
-// zero on entry. Returns false, with nothing emitted, when a bucket that
-// starts below `count` holds more than kSortBucketMax keys.
-template <typename Emit>
-__device__ __forceinline__ bool counting_sort_mask(FinishSort& fs, const uint64_t (&key)[kSortPerThread],
-                                                   uint32_t valid, uint32_t n, uint32_t lo,
-                                                   uint32_t hi, int count, Emit&& emit) {
+// One counting sort of the n candidate keys (unique composite keys) held
+// kSortPerThread per thread (slot j of a thread holds a key when bit j of
+// `valid` is set): kSortBins buckets, bucket_of(key) < kSortBins not falling
+// with the key, ranks inside a bucket by comparison, the first `count` <= n
+// through LDS to emit(i, key). Buckets that start at or past `count` hold no
+// output key and are neither ranked nor limited in size. fs.cursor and
+// fs.crowded must be zero on entry. Returns false, with nothing emitted, when
+// a bucket that starts below `count` holds more than kSortBucketMax keys.
+template <typename Bucket, typename Emit>
+__device__ __forceinline__ bool counting_sort_buckets(FinishSort& fs, const uint64_t (&key)[kSortPerThread],
+                                                      uint32_t valid, uint32_t n, Bucket&& bucket_of,
+                                                      int count, Emit&& emit) {
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
-  // Linear buckets over the radix keys [lo, hi], descending order =
-  // descending bucket, then descending key.
-  const uint32_t span = hi - lo + 1u;  // 0 stands for 2^32
-  const int bits = 32 - __builtin_clz((span - 1) | 1u);
-  const int shift = bits > 12 ? bits - 12 : 0;
-  // (Clamped: keys outside the range only come with counts that disagree
-  // with the scores, and must not index outside the buckets.)
-  auto bucket_of = [lo, shift](uint64_t k) {
-    return min(((uint32_t)(k >> 32) - lo) >> shift, (uint32_t)kSortBins - 1);
-  };
 #pragma unroll
   for (int j = 0; j < kSortPerThread; ++j)
     if ((valid >> j) & 1u) atomicAdd(&fs.cursor[bucket_of(key[j])], 1u);
@@ -1245,6 +1234,128 @@ __device__ __forceinline__ bool counting_sort_mask(FinishSort& fs, const uint64_
     return true;
   }
   return false;
+}
+
+// Linear buckets of the values between the radix keys `lo` and `hi` (finite):
+// false when their span or its reciprocal overflows. The steps round, but
+// none of them can order two values the wrong way.
+struct ValueBuckets {
+  float least, per;
+  __device__ __forceinline__ bool set(uint32_t lo, uint32_t hi) {
+    least = __uint_as_float(key_bits(lo));
+    const float span = __uint_as_float(key_bits(hi)) - least;
+    per = span > 0.0f ? (float)(kSortBins - 1) / span : 0.0f;
+    return span <= 1e37f && (span == 0.0f || span >= 1e-30f);
+  }
+  __device__ __forceinline__ uint32_t operator()(uint64_t k) const {
+    const float x = (__uint_as_float(key_bits((uint32_t)(k >> 32))) - least) * per;
+    return min((uint32_t)fmaxf(x, 0.0f), (uint32_t)kSortBins - 1);
+  }
+};
+
+__device__ __forceinline__ bool finite_key(uint32_t radix) {
+  return (key_bits(radix) & 0x7F800000u) != 0x7F800000u;
+}
+
+// The same for keys whose radix keys lie in [lo, hi]: buckets of the values,
+// or, where an end is not finite or the span extreme, of the radix keys.
+// (Radix buckets put most keys of a range that crosses zero - a row whose
+// threshold is negative, as of one in a few hundred at 64K columns, more at
+// fewer - into a few dozen buckets, too crowded to rank, and one such row sets
+// the launch: 128 rows x 65,664 columns 17.7 -> 9.2 us, 37 x 20,048 25.9 -> 9.1.)
+// Keys outside the range only come with counts that disagree with the
+// scores; they are clamped, so that they index no other memory.
+template <typename Emit>
+__device__ __forceinline__ bool counting_sort_mask(FinishSort& fs, const uint64_t (&key)[kSortPerThread],
+                                                   uint32_t valid, uint32_t n, uint32_t lo,
+                                                   uint32_t hi, int count, Emit&& emit) {
+  const uint32_t span = hi - lo + 1u;  // 0 stands for 2^32
+  const int bits = 32 - __builtin_clz((span - 1) | 1u);
+  const int shift = bits > 12 ? bits - 12 : 0;
+  ValueBuckets of_value;
+  const bool by_value = of_value.set(lo, hi) && finite_key(lo) && finite_key(hi);
+  auto bucket_of = [=](uint64_t k) -> uint32_t {
+    if (by_value) return of_value(k);
+    return min(((uint32_t)(k >> 32) - lo) >> shift, (uint32_t)kSortBins - 1);
+  };
+  return counting_sort_buckets(fs, key, valid, n, bucket_of, count, emit);
+}
+
+// The top `count` of a row of which at most kSortCap columns, [lo, hi), are
+// visible (the others are -inf): every finite score goes into one counting
+// sort over kSortBins linear buckets of the values between the row's smallest
+// and largest, then -inf / -1 slots. Returns false, with nothing written, for
+// a row with a NaN, +inf or an extreme span, or a crowded bucket (many
+// near-equal scores). The
+// work-group's threads call it together.
+template <typename Emit>
+__device__ __forceinline__ bool sort_visible(FinishSort& fs, uint4* __restrict__ wave_parts,
+                                             const float* __restrict__ row, int64_t lo, int64_t hi,
+                                             int count, Emit&& emit) {
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = tid >> 6;
+  constexpr int kWaves = kThreads / 64;
+  constexpr uint32_t kNegInf = 0xFF800000u;
+  uint64_t key[kSortPerThread];
+  float v[kSortPerThread];
+#pragma unroll
+  for (int j = 0; j < kSortPerThread; ++j) {
+    const int64_t c = lo + tid + j * kThreads;
+    v[j] = c < hi ? row[c] : __uint_as_float(kNegInf);
+  }
+  for (int i = tid; i < kSortBins; i += kThreads) fs.cursor[i] = 0;
+  if (tid == 0) fs.crowded = 0;
+  uint32_t valid = 0, largest = 0, smallest = 0xFFFFFFFFu, odd = 0;
+#pragma unroll
+  for (int j = 0; j < kSortPerThread; ++j) {
+    const uint32_t b = __float_as_uint(v[j]);
+    const bool finite = (b & 0x7F800000u) != 0x7F800000u;
+    if (!finite && b != kNegInf) odd = 1;
+    key[j] = composite(v[j], lo + tid + j * kThreads);
+    const uint32_t r = (uint32_t)(key[j] >> 32);
+    valid |= finite ? 1u << j : 0u;
+    largest = finite && r > largest ? r : largest;
+    smallest = finite && r < smallest ? r : smallest;
+  }
+  auto reduce = [&](auto m_tag) {
+    constexpr int kM = decltype(m_tag)::value;
+    const uint32_t a = lane_xor<kM>(largest), b = lane_xor<kM>(smallest);
+    largest = a > largest ? a : largest;
+    smallest = b < smallest ? b : smallest;
+  };
+  reduce(std::integral_constant<int, 1>{});
+  reduce(std::integral_constant<int, 2>{});
+  reduce(std::integral_constant<int, 4>{});
+  reduce(std::integral_constant<int, 8>{});
+  reduce(std::integral_constant<int, 16>{});
+  reduce(std::integral_constant<int, 32>{});
+  uint32_t total = 0;
+  (void)wave_prefix_any((uint32_t)__builtin_popcount(valid), &total);
+  const bool wave_odd = __builtin_amdgcn_ballot_w64(odd) != 0;
+  if (lane == 0) wave_parts[wave] = uint4{total, largest, smallest, wave_odd ? 1u : 0u};
+  __syncthreads();  // the wave parts and the LDS state above are set
+  uint32_t n = 0;
+  largest = 0;
+  smallest = 0xFFFFFFFFu;
+  odd = 0;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) {
+    const uint4 part = wave_parts[w];
+    n += part.x;
+    largest = part.y > largest ? part.y : largest;
+    smallest = part.z < smallest ? part.z : smallest;
+    odd |= part.w;
+  }
+  if (odd) return false;
+  const int found = n < (uint32_t)count ? (int)n : count;
+  if (found > 0) {
+    ValueBuckets bucket_of;
+    if (!bucket_of.set(smallest, largest)) return false;
+    if (!counting_sort_buckets(fs, key, valid, n, bucket_of, found, emit)) return false;
+  }
+  for (int i = found + tid; i < count; i += kThreads) emit(i, (uint64_t)0x007FFFFFu << 32);
+  return true;
 }
 
 // The same with the keys at positions t + j kThreads < n.
@@ -1415,6 +1526,12 @@ struct LogitsInputs {
 };
 constexpr int kMaxCandidateSplits = 512;
 
+// kShort: calls of at most kSortCap columns, whose rows have no floor unless
+// the caller gave one: a row stored in full is sorted at once (sort_visible),
+// and select_row is left with the rows that this refuses. Against select_row
+// for every row: 128 rows of 4,224 columns 30.1 -> 9.4 us, 2,048 rows of up to
+// 2,048 columns 129 -> 60 us.
+template <bool kShort>
 __global__ __launch_bounds__(kThreads, 1) void topk_candidates(float* __restrict__ scores,
                                                               int64_t cols, int64_t ld,
                                                               int total_count,
@@ -1467,13 +1584,14 @@ __global__ __launch_bounds__(kThreads, 1) void topk_candidates(float* __restrict
   asm volatile("" : "+v"(rec0), "+v"(rec1));
 #pragma unroll
   for (int j = 0; j < kSpecSlots; ++j) asm volatile("" : "+v"(key[j]));
-  if (floor == 0) {
-    select_row<kResidentVecSmall>(lds.sh, scores, cols, ld, total_count, values, ids, out_ld,
-                                  nullptr, r, 0, 1);
+  constexpr int kResident = kShort ? kSortCap / (4 * kThreads) : kResidentVecSmall;
+  if (floor == 0 && !kShort) {
+    select_row<kResident>(lds.sh, scores, cols, ld, total_count, values, ids, out_ld, nullptr, r, 0, 1);
     return;
   }
-  const int64_t vis_lo = li.starts ? (int64_t)li.starts[r] : 0;
+  int64_t vis_lo = li.starts ? (int64_t)li.starts[r] : 0;
   int64_t vis_hi = li.ends ? (int64_t)li.ends[r] : li.query_start + r + 1;
+  if (kShort && vis_lo < 0) vis_lo = 0;
   if (vis_hi > cols) vis_hi = cols;
   float* row = scores + r * ld;
   float* vout = values + r * out_ld;
@@ -1484,6 +1602,12 @@ __global__ __launch_bounds__(kThreads, 1) void topk_candidates(float* __restrict
     const bool finite = (b & 0x7F800000u) != 0x7F800000u;
     iout[i] = finite ? (int32_t)(~(uint32_t)k) : -1;
   };
+  if (kShort && floor == 0) {
+    if (sort_visible(fs, wave_parts, row, vis_lo, vis_hi, count, emit)) return;
+    __syncthreads();
+    select_row<kResident>(lds.sh, scores, cols, ld, total_count, values, ids, out_ld, nullptr, r, 0, 1);
+    return;
+  }
   for (int i = tid; i < kSortBins; i += kThreads) fs.cursor[i] = 0;
   if (tid == 0) fs.crowded = 0;
 
@@ -1750,7 +1874,7 @@ __global__ __launch_bounds__(kThreads, 1) void topk_candidates(float* __restrict
   logits_core::row_scores(li.q, li.k, li.w, li.kscale, li.q_fold, r, (int32_t)vis_lo,
                           (int32_t)vis_hi, cols, row, digits, wave, kThreads / 64);
   __syncthreads();
-  select_row<kResidentVecSmall>(lds.sh, scores, cols, ld, total_count, values, ids, out_ld,
+  select_row<kResident>(lds.sh, scores, cols, ld, total_count, values, ids, out_ld,
                                 nullptr, r, 0, 1);
 }
 }  // namespace
@@ -1832,8 +1956,8 @@ int topk_from_candidates(const uint8_t* q, const uint8_t* k, const float* weight
   DSA_CHECK_ARG(splits >= 1 && splits <= kMaxCandidateSplits, "too many key splits");
   DSA_CHECK_ARG(columns < (int64_t)0x7FFFFFFF && rows < 0x7FFFFFFF, "too many rows or columns");
   const int64_t count = topk < columns ? topk : columns;
-  hipLaunchKernelGGL(topk_candidates, dim3((unsigned)rows), dim3(kThreads), 0, stream, scores,
-                     columns, ld, (int)count, values, indices, out_ld,
+  hipLaunchKernelGGL((columns <= kSortCap ? topk_candidates<true> : topk_candidates<false>),
+                     dim3((unsigned)rows), dim3(kThreads), 0, stream, scores, columns, ld, (int)count, values, indices, out_ld,
                      CandidateLists{floors, records, lists, splits, per, cap},
                      LogitsInputs{q, k, weights, kscale, starts, ends, query_start, q_fold});
   DSA_CHECK_LAUNCH("indexer top-k from candidates");
