@@ -6,7 +6,8 @@ operator.
 """
 
 import ctypes
-from functools import cache
+from contextlib import nullcontext
+from functools import cache, lru_cache
 from pathlib import Path
 
 import torch
@@ -55,6 +56,9 @@ SIGNATURES = {
     "dsa_layer_prologue_floors_fp8": [_ptr, _i64, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _ptr,
                                       _ptr, _ptr, _i64, _i64, _ptr, _i64, _ptr, _ptr, _ptr, _ptr,
                                       _i64, _i64, _ptr, _ptr],
+    "dsa_layer_indexer_scratch_bytes": [_i64, _i64, _i64, ctypes.POINTER(ctypes.c_int64)],
+    "dsa_layer_indexer_fp8": [_ptr, _i64, _ptr, _ptr, _ptr, _ptr, _i64, _ptr, _ptr, _ptr, _i64,
+                              _i64, _ptr, _ptr, _ptr, _i64, _ptr, _i64, _ptr],
     "dsa_index_producer_fp8": [_ptr, _i64, _ptr, _f32, _f32, _ptr, _ptr, _ptr, _f32, _ptr, _i64,
                                _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _ptr, _i64,
                                _ptr, _ptr, _ptr],
@@ -113,8 +117,16 @@ def last_error():
     return buf.value.decode(errors="replace")
 
 
+# Entry points by name, filled at their first call (a lookup on the library
+# object costs as much as a short call).
+_ENTRIES = {}
+
+
 def call(name, *args):
-    status = getattr(library(), name)(*args)
+    entry = _ENTRIES.get(name)
+    if entry is None:
+        entry = _ENTRIES[name] = getattr(library(), name)
+    status = entry(*args)
     if status != 0:
         message = last_error()
         if status == 1:
@@ -122,19 +134,51 @@ def call(name, *args):
         raise NativeError(f"{name} failed ({status}): {message}")
 
 
+@lru_cache(maxsize=1024)
+def size_of(name, device_index, *args):
+    """The byte count a ``*_bytes`` entry point gives for ``args`` on a device
+    (the current one): a function of the shapes and the device's CU count."""
+    needed = ctypes.c_int64()
+    call(name, *args, ctypes.byref(needed))
+    return needed.value
+
+
 def ptr(tensor):
     """Device (or host) address of a tensor, or None for a missing tensor."""
-    return None if tensor is None else ctypes.c_void_p(tensor.data_ptr())
+    return None if tensor is None else tensor.data_ptr()
+
+
+def raw_stream(device):
+    """Address of the device's current stream (0: the default stream)."""
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 def stream_of(device):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    return ctypes.c_void_p(raw_stream(device))
+
+
+_CURRENT = nullcontext()
+
+
+def on_device(device):
+    """``torch.cuda.device(device)``, or nothing when it is current already."""
+    if device.index is not None and torch.cuda.current_device() == device.index:
+        return _CURRENT
+    return torch.cuda.device(device)
+
+
+_GFX950 = set()  # device indices known to be gfx950
 
 
 def require_gfx950(device, what):
     """The native kernels are built for gfx950 only."""
+    if device.type == "cuda" and device.index in _GFX950:
+        return
     if device.type != "cuda" or not torch.cuda.is_available():
         raise NotImplementedError(f"{what} requires an MI355X (gfx950) HIP device")
     arch = torch.cuda.get_device_properties(device).gcnArchName.split(":")[0]
     if arch != "gfx950":
         raise NotImplementedError(f"{what} requires an MI355X (gfx950) HIP device, got {arch}")
+    if device.index is not None:
+        _GFX950.add(device.index)

@@ -18,7 +18,6 @@ padding semantics and validation messages):
 Kernels: ``csrc/sparse_mla.hip`` and ``csrc/quantize.hip``.
 """
 
-import ctypes
 import math
 
 import torch
@@ -77,10 +76,9 @@ def _narrow_ids(indices, limit):
 def _workspace(q, selected):
     """The kernel's workspace for this call (None when it needs none), from
     torch's allocator on the current stream, on which the kernels read it."""
-    needed = ctypes.c_int64()
-    _native.call("dsa_sparse_mla_workspace_bytes", q.shape[0], q.shape[1], selected,
-                 ctypes.byref(needed))
-    return torch.empty(needed.value, dtype=torch.uint8, device=q.device) if needed.value else None
+    needed = _native.size_of("dsa_sparse_mla_workspace_bytes", q.device.index, q.shape[0],
+                             q.shape[1], selected)
+    return torch.empty(needed, dtype=torch.uint8, device=q.device) if needed else None
 
 
 def sparse_mla(q, kv, indices, scale, value_dim=512):
@@ -99,7 +97,7 @@ def sparse_mla(q, kv, indices, scale, value_dim=512):
     out = torch.empty((*q.shape[:2], value_dim), dtype=q.dtype, device=q.device)
     q, kv = _aligned(q), _aligned(kv)
     ids = _narrow_ids(indices, kv.shape[0])
-    with torch.cuda.device(q.device):
+    with _native.on_device(q.device):
         workspace = _workspace(q, ids.shape[1])
         _native.call(
             "dsa_sparse_mla_bf16_ws",
@@ -180,7 +178,7 @@ def sparse_mla_fp8_paged(q, kv_cache, page_table, indices, scale, value_dim=512,
     cache = _aligned(kv_cache)
     table = page_table.contiguous()
     ids = _narrow_ids(indices, n_tokens)
-    with torch.cuda.device(q.device):
+    with _native.on_device(q.device):
         workspace = _workspace(q, ids.shape[1])
         _native.call(
             "dsa_sparse_mla_fp8_paged_ws",
@@ -220,7 +218,7 @@ def pack_kv_fp8(kv, kv_cache, page_table, token_offset=0, status=None):
     kv = _aligned(kv)
     if kv_cache.data_ptr() % 16:
         raise ValueError("kv_cache must be 16-byte aligned")
-    with torch.cuda.device(kv.device):
+    with _native.on_device(kv.device):
         _native.call(
             "dsa_kv_pack_fp8",
             _native.ptr(kv), tokens, token_offset,

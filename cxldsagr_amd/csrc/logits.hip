@@ -973,3 +973,69 @@ extern "C" int dsa_indexer_select_fp8(const void* q, const void* k, const float*
                                q_fold, scores, topk, values, indices, out_ld, 0, workspace,
                                workspace_bytes, stream);
 }
+
+// A layer step's indexer half in one call: the prologue launch with floors,
+// the candidate logits and their top-k, over one scratch for what only the
+// three share (q codes, scales, folded weights and queries, top-k values).
+namespace dsa {
+namespace {
+struct IndexerScratch {
+  int64_t scales, folded, fold, values, bytes;
+};
+IndexerScratch indexer_scratch(int64_t rows, int64_t count) {
+  IndexerScratch s;
+  s.scales = rows * kHeads * kDim;
+  s.folded = s.scales + rows * kHeads * 4;
+  s.fold = s.folded + rows * kHeads * 4;
+  s.values = s.fold + rows * 4 * kDim * 4;
+  s.bytes = s.values + rows * count * 4;
+  return s;
+}
+}  // namespace
+}  // namespace dsa
+
+extern "C" int dsa_layer_indexer_scratch_bytes(int64_t rows, int64_t columns, int64_t topk,
+                                               int64_t* bytes) {
+  using namespace dsa;
+  DSA_CHECK_ARG(rows >= 0 && rows < 0x7FFFFFFF && columns >= 1 && topk >= 1 && topk <= 2048 &&
+                    bytes != nullptr,
+                "invalid layer indexer scratch query");
+  *bytes = indexer_scratch(rows, topk < columns ? topk : columns).bytes;
+  return kOk;
+}
+
+extern "C" int dsa_layer_indexer_fp8(const void* q, int64_t rows, const float* weights,
+                                     const void* k, const void* kv, const int32_t* page_table,
+                                     int64_t pages, void* cache, void* index_keys,
+                                     float* index_scales, int64_t position, int64_t topk,
+                                     int32_t* indices, float* scores, void* scratch,
+                                     int64_t scratch_bytes, void* workspace,
+                                     int64_t workspace_bytes, hipStream_t stream) {
+  using namespace dsa;
+  DSA_CHECK_ARG(rows >= 1 && position >= 0 && topk >= 1 && topk <= 2048, "invalid layer indexer shape");
+  DSA_CHECK_ARG(index_keys && index_scales && indices, "null pointer");
+  const int64_t columns = position + rows;
+  const int64_t count = topk < columns ? topk : columns;
+  const IndexerScratch at = indexer_scratch(rows, count);
+  DSA_CHECK_ARG(scratch != nullptr && reinterpret_cast<uintptr_t>(scratch) % 16 == 0 &&
+                    scratch_bytes >= at.bytes,
+                "layer indexer scratch too small or misaligned");
+  uint8_t* base = static_cast<uint8_t*>(scratch);
+  float* folded = reinterpret_cast<float*>(base + at.folded);
+  float* q_fold = reinterpret_cast<float*>(base + at.fold);
+  int status = dsa_layer_prologue_floors_fp8(
+      q, rows * kHeads, weights, base, reinterpret_cast<float*>(base + at.scales), folded, q_fold, k,
+      rows, static_cast<uint8_t*>(index_keys) + position * kDim, index_scales + position, kv,
+      kv ? rows : 0, kv ? position : 0, page_table, kv ? pages : 0, cache, nullptr, index_keys,
+      index_scales, position, topk, static_cast<uint32_t*>(workspace), stream);
+  if (status != kOk) return status;
+  const int64_t ldo = (columns + 255) / 256 * 256;
+  status = dsa_indexer_logits_fp8_emit(base, index_keys, folded, index_scales, nullptr, nullptr,
+                                       position, rows, columns, ldo, q_fold, scores, 0, workspace,
+                                       workspace_bytes, stream);
+  if (status != kOk) return status;
+  return dsa_indexer_emit_topk(base, index_keys, folded, index_scales, nullptr, nullptr, position,
+                               rows, columns, q_fold, scores, topk,
+                               reinterpret_cast<float*>(base + at.values), indices, count, 0,
+                               workspace, workspace_bytes, stream);
+}

@@ -109,7 +109,7 @@ def _quantize(x, scale_fmt, weights):
         _native.ptr(scales),
         1 if scale_fmt == "ue8m0" else 0,
     )
-    with torch.cuda.device(x.device):
+    with _native.on_device(x.device):
         if weights is None:
             _native.call("dsa_quantize_fp8_rows", *common, _native.stream_of(x.device))
         else:
@@ -137,7 +137,7 @@ def quantize_into(x, codes, scales, scale_fmt="ue8m0"):
     _native.require_gfx950(x.device, "indexer quantization")
     if rows == 0:
         return codes, scales
-    with torch.cuda.device(x.device):
+    with _native.on_device(x.device):
         _native.call(
             "dsa_quantize_fp8_rows", _native.ptr(x), _native.DTYPE_CODES[x.dtype], rows, dim,
             x.stride(0), _native.ptr(codes), _native.ptr(scales),
@@ -173,7 +173,7 @@ def logits(q, k, weights, kscale, query_start, prefetch=None, *, _bounds=None,
     args, q_fold, output, _operands = _logits_launch_args(q, k, weights, kscale, query_start,
                                                           _bounds, _q_fold)
     device = q.device
-    with torch.cuda.device(device):
+    with _native.on_device(device):
         if q_fold is None:
             _native.call("dsa_indexer_logits_fp8", *args, _native.ptr(output),
                          _native.stream_of(device))
@@ -203,7 +203,7 @@ def logits_topk(q, k, weights, kscale, query_start, topk, *, _bounds=None, _q_fo
     count = min(topk, columns)
     values = torch.empty((rows, count), dtype=torch.float32, device=device)
     indices = torch.empty((rows, count), dtype=torch.int32, device=device)
-    with torch.cuda.device(device):
+    with _native.on_device(device):
         stream = _native.stream_of(device)
         workspace = _digit_workspace(device, stream, rows, columns)
         _native.call("dsa_indexer_topk_fp8", *args, _native.ptr(q_fold), _native.ptr(scores), topk,
@@ -245,7 +245,7 @@ def select_topk(q, k, weights, kscale, query_start, topk, *, _bounds=None, _q_fo
     values = torch.empty((rows, count), dtype=torch.float32, device=device)
     indices = torch.empty((rows, count), dtype=torch.int32, device=device)
     head = args[:9]  # q, k, weights, kscale, starts, ends, query_start, rows, columns
-    with torch.cuda.device(device):
+    with _native.on_device(device):
         stream = _native.stream_of(device)
         workspace, scores = _select_buffers(device, stream, rows, columns, _list_cap)
         if _floors is None and _list_cap == 0 and not _floors_ready:
@@ -268,13 +268,39 @@ def select_topk(q, k, weights, kscale, query_start, topk, *, _bounds=None, _q_fo
     return values, indices
 
 
+def layer_select(index_q, index_k, weights, index_keys, index_scales, position, topk, *, kv=None,
+                 page_table=None, kv_cache=None):
+    """A layer step's indexer in one native call (``dsa_layer_indexer_fp8``: the
+    prologue launch with floors, the candidate logits, their top-k): the int32
+    ids ``[rows, min(topk, position + rows)]``, as ``index_prologue`` and
+    ``select_topk`` give them. Inputs as those take them, contiguous and
+    16-byte aligned; the caches whole."""
+    device, rows = index_q.device, len(index_q)
+    columns = position + rows
+    with _native.on_device(device):
+        stream = _native.stream_of(device)
+        workspace, scores = _select_buffers(device, stream, rows, columns, 0)
+        needed = _native.size_of("dsa_layer_indexer_scratch_bytes", device.index, rows, columns, topk)
+        scratch = torch.empty(needed, dtype=torch.uint8, device=device)
+        ids = torch.empty((rows, min(topk, columns)), dtype=torch.int32, device=device)
+        paged = kv is not None
+        _native.call(
+            "dsa_layer_indexer_fp8", index_q.data_ptr(), rows, weights.data_ptr(),
+            index_k.data_ptr(), _native.ptr(kv), _native.ptr(page_table if paged else None),
+            kv_cache.shape[0] if paged else 0, _native.ptr(kv_cache if paged else None),
+            index_keys.data_ptr(), index_scales.data_ptr(), position, topk, ids.data_ptr(),
+            scores.data_ptr(), scratch.data_ptr(), needed, workspace.data_ptr(),
+            workspace.numel(), stream)
+    return ids
+
+
 def select_floors_buffer(device, rows, columns):
     """The floors (int32 ``[rows, 2]``: two estimates per row, the row's floor
     being the smaller as uint32) of the current stream's ``select_topk``
     workspace for ``rows`` x ``columns``: a producer that computes the floors
     itself (``dsa_layer_prologue_floors_fp8``) writes them here, then calls
     ``select_topk(..., _floors_ready=True)``."""
-    with torch.cuda.device(device):
+    with _native.on_device(device):
         workspace, _ = _select_buffers(device, _native.stream_of(device), rows, columns, 0)
     return workspace[:8 * rows].view(torch.int32).view(rows, 2)
 
@@ -285,7 +311,7 @@ def select_floors(q, k, weights, kscale, query_start, topk, *, _bounds=None):
     args, _, _, _operands = _logits_launch_args(q, k, weights, kscale, query_start, _bounds, None,
                                                 allocate_output=False)
     floors = torch.empty((len(q), 2), dtype=torch.int32, device=q.device)
-    with torch.cuda.device(q.device):
+    with _native.on_device(q.device):
         _native.call("dsa_indexer_floors_fp8", *args[:9], topk, _native.ptr(floors),
                      _native.stream_of(q.device))
     return floors[:, 0].contiguous()
@@ -362,7 +388,7 @@ def exact_topk(scores, k):
         return values, indices
     if scores.stride(1) != 1 or scores.stride(0) < columns:
         scores = scores.contiguous()
-    with torch.cuda.device(device):
+    with _native.on_device(device):
         stream = _native.stream_of(device)
         workspace = _topk_workspace(device, stream, rows)
         _native.call(
@@ -417,25 +443,23 @@ _SELECT_BUFFERS = {}
 def _select_buffers(device, stream, rows, columns, list_cap):
     key = (device.index, stream.value)
     workspace, scores = _SELECT_BUFFERS.get(key, (None, None))
-    needed = ctypes.c_int64()
-    _native.call("dsa_indexer_select_workspace_bytes", rows, columns, list_cap,
-                 ctypes.byref(needed))
-    if workspace is None or workspace.numel() < needed.value:
+    needed = _native.size_of("dsa_indexer_select_workspace_bytes", device.index, rows, columns,
+                             list_cap)
+    if workspace is None or workspace.numel() < needed:
         # 256-byte alignment: the caching allocator's blocks are 512-aligned.
-        workspace = torch.empty(needed.value, dtype=torch.uint8, device=device)
+        workspace = torch.empty(needed, dtype=torch.uint8, device=device)
     width = padded_columns(columns)
     if scores is None or scores.numel() < rows * width:
         scores = torch.empty(rows * width, dtype=torch.float32, device=device)
     _SELECT_BUFFERS[key] = (workspace, scores)
-    return workspace, scores[:rows * width].view(rows, width)
+    return workspace, torch.as_strided(scores, (rows, width), (width, 1))
 
 
 def _topk_workspace(device, stream, rows):
     key = (device.index, stream.value)
     workspace = _TOPK_WORKSPACES.get(key)
-    needed = ctypes.c_int64()
-    _native.call("dsa_topk_workspace_bytes", rows, ctypes.byref(needed))
-    if workspace is None or workspace.numel() < needed.value:
-        workspace = torch.empty(needed.value, dtype=torch.uint8, device=device)
+    needed = _native.size_of("dsa_topk_workspace_bytes", device.index, rows)
+    if workspace is None or workspace.numel() < needed:
+        workspace = torch.empty(needed, dtype=torch.uint8, device=device)
         _TOPK_WORKSPACES[key] = workspace
     return workspace

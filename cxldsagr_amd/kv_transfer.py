@@ -82,7 +82,7 @@ def gather_host_records(host, device, host_ids, device_ids, *, max_ctas=None, va
     if status is None:
         status = _status_word(device.device)
     kind = 1 if valid_count is not None and valid_count.dtype == torch.uint32 else 0
-    with torch.cuda.device(device.device):
+    with _native.on_device(device.device):
         _native.call(
             "dsa_gather_records",
             _native.ptr(host), host.shape[0],
@@ -120,7 +120,7 @@ def copy_host_records_async(host, device, *, host_start, device_start, count):
     if not count:
         return
     row_bytes = host.shape[1] * host.element_size()
-    with torch.cuda.device(device.device):
+    with _native.on_device(device.device):
         _native.call(
             "dsa_copy_records_h2d",
             _native.ptr(host[host_start:]),

@@ -40,6 +40,30 @@ def index_prologue_applies(index_q, index_k, weights, device):
             and all(t.device == device for t in (index_q, index_k, weights)))
 
 
+def _one_call_select(layer, index_q, index_k, weights, position, kv=None):
+    """The ids of ``indexer.layer_select`` for a batch the one-launch prologue
+    covers, or None where its inputs or caches want the checks and copies of
+    the separate operators. ``kv`` goes into the fp8 paged cache as well."""
+    rows = len(index_q)
+    keys, scales = layer.index_keys, layer.index_scales
+    if (not rows or type(layer.topk) is not int or not 1 <= layer.topk <= 2048
+            or type(position) is not int or not index_prologue_applies(index_q, index_k, weights, layer.device)
+            or keys.dtype != torch.float8_e4m3fn or scales.dtype != torch.float32
+            or len(keys) < position + rows or len(scales) < position + rows
+            or not (keys.is_contiguous() and scales.is_contiguous()) or keys.data_ptr() % 16
+            or keys.requires_grad or scales.requires_grad
+            or keys.device != index_q.device or scales.device != index_q.device):
+        return None
+    index_q, index_k, weights = (attention._aligned(t) for t in (index_q, index_k, weights))
+    if kv is None:
+        return indexer.layer_select(index_q, index_k, weights, keys, scales, position, layer.topk)
+    if not layer.kv_cache.is_contiguous() or not layer.page_table.is_contiguous():
+        return None
+    return indexer.layer_select(index_q, index_k, weights, keys, scales, position, layer.topk,
+                                kv=attention._aligned(kv), page_table=layer.page_table,
+                                kv_cache=layer.kv_cache)
+
+
 def index_prologue(index_q, index_k, weights, index_keys, index_scales, position, topk, floors,
                    *, kv=None, page_table=None, kv_cache=None):
     """The small stages before the indexer's logits in one launch
@@ -61,7 +85,7 @@ def index_prologue(index_q, index_k, weights, index_keys, index_scales, position
     q_fold = torch.empty((rows, 4, 128), dtype=torch.float32, device=device)
     if kv is not None:
         kv = attention._aligned(kv.contiguous())
-    with torch.cuda.device(device):
+    with _native.on_device(device):
         _native.call(
             "dsa_layer_prologue_floors_fp8",
             _native.ptr(index_q), rows * 64, _native.ptr(weights), _native.ptr(q8),
@@ -154,13 +178,8 @@ class DSALayer:
         end = position + rows
         if end > self.capacity:
             raise ValueError("query batch exceeds the layer capacity")
-        if index_prologue_applies(index_q, index_k, weights, self.device):
-            floors = indexer.select_floors_buffer(self.device, rows, end)
-            q8, folded, q_fold = index_prologue(index_q, index_k, weights, self.index_keys,
-                                                self.index_scales, position, self.topk, floors)
-            _, ids = indexer.select_topk(q8, self.index_keys[:end], folded,
-                                         self.index_scales[:end], position, self.topk,
-                                         _q_fold=q_fold, _floors_ready=True)
+        ids = _one_call_select(self, index_q, index_k, weights, position)
+        if ids is not None:
             return TokenSelection(ids)
         q8, _, weights = indexer.quantize_index_folded(index_q, weights)
         indexer.quantize_into(index_k, self.index_keys[position:end],
@@ -210,23 +229,18 @@ class DSALayer:
         end = position + rows
         if end > self.capacity or len(q) != rows or len(kv) != rows or len(index_k) != rows:
             raise ValueError("query batch exceeds the layer capacity or inputs disagree in length")
-        q_fold = floors = None
-        if self._fused_prologue_applies(index_q, index_k, weights, kv):
-            floors = indexer.select_floors_buffer(self.device, rows, end)
-            q8, folded, q_fold = self._prologue(index_q, index_k, weights, kv, position, floors)
-        elif index_prologue_applies(index_q, index_k, weights, self.device):
-            floors = indexer.select_floors_buffer(self.device, rows, end)
-            q8, folded, q_fold = index_prologue(index_q, index_k, weights, self.index_keys,
-                                                self.index_scales, position, self.topk, floors)
-            self._append_kv(kv, position)
-        else:
+        paged = (self.kv_format == "fp8_paged" and kv.dtype == torch.bfloat16
+                 and tuple(kv.shape) == (rows, attention.QK_DIM) and kv.device == index_q.device)
+        ids = _one_call_select(self, index_q, index_k, weights, position, kv if paged else None)
+        if ids is None:
             indexer.quantize_into(index_k, self.index_keys[position:end],
                                   self.index_scales[position:end])
             q8, _, folded = indexer.quantize_index_folded(index_q, weights)
             self._append_kv(kv, position)
-        _, ids = indexer.select_topk(q8, self.index_keys[:end], folded,
-                                     self.index_scales[:end], position, self.topk,
-                                     _q_fold=q_fold, _floors_ready=floors is not None)
+            _, ids = indexer.select_topk(q8, self.index_keys[:end], folded,
+                                         self.index_scales[:end], position, self.topk)
+        elif not paged:
+            self._append_kv(kv, position)
         selection = TokenSelection(ids)
         out = self._attend(q, ids, end)
         self.written = end
@@ -344,15 +358,8 @@ class OffloadDSALayer:
         end = position + len(index_q)
         if end > self.capacity or len(index_k) != len(index_q) or len(weights) != len(index_q):
             raise ValueError("query batch exceeds the layer capacity or inputs disagree in length")
-        rows = len(index_q)
-        if index_prologue_applies(index_q, index_k, weights, self.device):
-            # Quantisers and the candidate top-k's floors in one launch.
-            floors = indexer.select_floors_buffer(self.device, rows, end)
-            q8, folded, q_fold = index_prologue(index_q, index_k, weights, self.index_keys,
-                                                self.index_scales, position, self.topk, floors)
-            _, ids = indexer.select_topk(q8, self.index_keys[:end], folded,
-                                         self.index_scales[:end], position, self.topk,
-                                         _q_fold=q_fold, _floors_ready=True)
+        ids = _one_call_select(self, index_q, index_k, weights, position)
+        if ids is not None:
             return ids
         q8, _, folded = indexer.quantize_index_folded(index_q, weights)
         indexer.quantize_into(index_k, self.index_keys[position:end], self.index_scales[position:end])

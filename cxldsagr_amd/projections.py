@@ -183,7 +183,7 @@ def index_producer(q_proj, k_proj, head_logits, norm_weight, norm_bias, eps, cos
     if tokens == 0:
         return q8, q_scales, weights, index_keys, index_scales, fold
     pre, post = head_scales
-    with torch.cuda.device(device):
+    with _native.on_device(device):
         _native.call(
             "dsa_index_producer_floors_fp8" if floor_args else "dsa_index_producer_fp8",
             _native.ptr(q_proj), tokens, _native.ptr(head_logits), float(pre), float(post),

@@ -126,7 +126,7 @@ class TokenPool:
             kv = kv_bf16.contiguous()
             if kv.data_ptr() % 16:
                 kv = kv.clone()
-            with torch.cuda.device(self.device):
+            with _native.on_device(self.device):
                 _native.call("dsa_kv_pack_fp8", _native.ptr(kv), len(kv), start,
                              _native.ptr(session.page_table), self.host_capacity // PAGE_SIZE,
                              _native.ptr(self.host), _native.ptr(self.status),
@@ -142,7 +142,7 @@ class TokenPool:
         stale residency. Synchronises the current stream (the pool must be
         quiescent, as in the reference)."""
         self._check_live(session)
-        with torch.cuda.device(self.device):
+        with _native.on_device(self.device):
             _native.call("dsa_pool_release_rows", _native.ptr(session.page_table),
                          len(session.host_pages), self.host_capacity, _native.ptr(self.h2d),
                          _native.ptr(self.d2h), _native.ptr(self.priority), self.slots,
@@ -234,7 +234,7 @@ class TokenPool:
             tail = (_native.stream_of(self.device), gather)
         else:
             tail = (_native.stream_of(self.device),)
-        with torch.cuda.device(self.device):
+        with _native.on_device(self.device):
             _native.call(
                 "dsa_pool_recall_pipelined" if pipelined else "dsa_pool_recall",
                 _native.ptr(ids), ids.numel(), _native.ptr(session.page_table),

@@ -327,6 +327,24 @@ int dsa_layer_prologue_floors_fp8(const void* q, int64_t q_rows, const float* we
                                   uint32_t* floors, hipStream_t stream);
 
 /*
+ * The indexer half of a layer step in one call:
+ * dsa_layer_prologue_floors_fp8 for `rows` queries at positions position ..,
+ * dsa_indexer_logits_fp8_emit and dsa_indexer_emit_topk over the
+ * position + rows resident keys; `indices` int32 [rows, min(topk, position +
+ * rows)]. index_keys e4m3 [>= position + rows, 128] / index_scales f32 are the
+ * whole cache (the new rows are written). kv (and page_table, pages, cache) is
+ * optional. `scores` and `workspace` as dsa_indexer_emit_topk takes them (the
+ * floors are written into the workspace); `scratch`, 16-byte aligned,
+ * dsa_layer_indexer_scratch_bytes bytes, needs no initialisation.
+ */
+int dsa_layer_indexer_scratch_bytes(int64_t rows, int64_t columns, int64_t topk, int64_t* bytes);
+int dsa_layer_indexer_fp8(const void* q, int64_t rows, const float* weights, const void* k,
+                          const void* kv, const int32_t* page_table, int64_t pages, void* cache,
+                          void* index_keys, float* index_scales, int64_t position, int64_t topk,
+                          int32_t* indices, float* scores, void* scratch, int64_t scratch_bytes,
+                          void* workspace, int64_t workspace_bytes, hipStream_t stream);
+
+/*
  * Indexer input producers: the indexer half of the projection step after
  * its GEMMs, in one launch. Replaces, in the reference's project()
  * (models/deepseek_v32/projections.py:182-257), the K LayerNorm of
