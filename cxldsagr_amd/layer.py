@@ -40,6 +40,34 @@ def index_prologue_applies(index_q, index_k, weights, device):
             and all(t.device == device for t in (index_q, index_k, weights)))
 
 
+def _one_launch_history(layer, index_k, kv, start, end):
+    """Quantise history rows (bf16 index K ``[rows, 128]``, KV ``[rows, 576]``)
+    into the key cache and the fp8 paged cache in one launch, a prologue
+    without queries. False, with nothing done, where the rows or the caches
+    want the checks of the separate operators."""
+    keys, scales, cache, table = layer.index_keys, layer.index_scales, layer.kv_cache, layer.page_table
+    if (start == end or index_k.dtype != torch.bfloat16 or index_k.ndim != 2
+            or index_k.shape[1] != 128 or index_k.stride(1) != 1
+            or kv.dtype != torch.bfloat16 or tuple(kv.shape) != (end - start, attention.QK_DIM)
+            or keys.dtype != torch.float8_e4m3fn or scales.dtype != torch.float32
+            or len(keys) < end or len(scales) < end or tuple(keys.shape[1:]) != (128,)
+            or not (keys.is_contiguous() and scales.is_contiguous()) or keys.data_ptr() % 16
+            or not (cache.is_contiguous() and table.is_contiguous()) or cache.data_ptr() % 16
+            or end > table.numel() * PAGE_TOKENS or not index_k.is_cuda
+            or any(t.device != index_k.device for t in (kv, keys, scales))):
+        return False
+    attention._check_paged(cache, table, kv.device)
+    index_k, kv = attention._aligned(index_k), attention._aligned(kv)
+    _native.require_gfx950(kv.device, "history write")
+    with _native.on_device(kv.device):
+        _native.call(
+            "dsa_layer_prologue_fp8", None, 0, None, None, None, None, None,
+            index_k.data_ptr(), end - start, keys[start:].data_ptr(), scales[start:].data_ptr(),
+            kv.data_ptr(), end - start, start, table.data_ptr(), cache.shape[0], cache.data_ptr(),
+            None, _native.stream_of(kv.device))
+    return True
+
+
 def _one_call_select(layer, index_q, index_k, weights, position, kv=None):
     """The ids of ``indexer.layer_select`` for a batch the one-launch prologue
     covers, or None where its inputs or caches want the checks and copies of
@@ -166,8 +194,9 @@ class DSALayer:
         start, end = self.written, self.written + len(index_k)
         if len(kv) != len(index_k) or end > self.capacity:
             raise ValueError("history exceeds the layer capacity or K/KV lengths differ")
-        indexer.quantize_into(index_k, self.index_keys[start:end], self.index_scales[start:end])
-        self._append_kv(kv, start)
+        if not (self.kv_format == "fp8_paged" and _one_launch_history(self, index_k, kv, start, end)):
+            indexer.quantize_into(index_k, self.index_keys[start:end], self.index_scales[start:end])
+            self._append_kv(kv, start)
         self.written = end
         return start
 
