@@ -709,17 +709,27 @@ __global__ __launch_bounds__(kThreads, 1) void sparse_mla_fwd(
     // ---- row sums of all 64 heads, then O / l.
     if (g == 0) lds.row_sum[16 * wave + c] = l_acc[0];
     __syncthreads();
-    uint16_t* obase = out + ((row * heads + head0 + c) * kVDim) + dim0 + 4 * g;
+    // Two dim tiles at a time: the row groups swap halves, so that a lane
+    // holds 8 consecutive dims (of tile m + (g & 1)) and a head's 64 bytes go
+    // out in one instruction. With 8 bytes a lane (32 of a head) the stores
+    // took 7.5k cycles to land, now 3.9k (1,024 rows of 128 heads and 2,048
+    // keys: 621 -> 610 us, 64 keys: 104 -> 92 us).
+    uint16_t* obase = out + ((row * heads + head0 + c) * kVDim) + dim0 + 16 * (g & 1) + 8 * (g >> 1);
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       const float lt = lds.row_sum[16 * t + c];
       const float inv_l = lt > 0.0f ? 1.0f / lt : 0.0f;
       uint16_t* orow = obase + (int64_t)16 * t * kVDim;
 #pragma unroll
-      for (int m = 0; m < kM; ++m)
-        *reinterpret_cast<uint2*>(orow + 16 * m) =
-            make_uint2(pack_bf16(o[t][m][0] * inv_l, o[t][m][1] * inv_l),
-                       pack_bf16(o[t][m][2] * inv_l, o[t][m][3] * inv_l));
+      for (int m = 0; m < kM; m += 2) {
+        const auto lo = __builtin_amdgcn_permlane16_swap(
+            pack_bf16(o[t][m][0] * inv_l, o[t][m][1] * inv_l),
+            pack_bf16(o[t][m + 1][0] * inv_l, o[t][m + 1][1] * inv_l), false, false);
+        const auto hi = __builtin_amdgcn_permlane16_swap(
+            pack_bf16(o[t][m][2] * inv_l, o[t][m][3] * inv_l),
+            pack_bf16(o[t][m + 1][2] * inv_l, o[t][m + 1][3] * inv_l), false, false);
+        *reinterpret_cast<uint4*>(orow + 16 * m) = make_uint4(lo[0], hi[0], lo[1], hi[1]);
+      }
     }
   };
   if (scorer) run(std::true_type{});
