@@ -1204,7 +1204,7 @@ __global__ __launch_bounds__(kValueThreads, kDv < 256 ? 2 : 1) void mla_values(
 // How a call's rows are run: rows [0, wide_rows) by sparse_mla_fwd, the rest in
 // the split form with kDv = dv.
 //
-// sparse_mla_fwd takes about 78 us (2,048 selected) for each round of one
+// sparse_mla_fwd takes about 76 us (2,048 selected) for each round of one
 // (row, 64 heads) work-group per CU, however few there are. The split form,
 // whose scores go through memory instead of LDS, measured 35 / 43 / 54 / 77 us
 // for 4 / 16 / 32 / 64 rows of 128 heads over 2,048 fp8 records (56 / 92 us
