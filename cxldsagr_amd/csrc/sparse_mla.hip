@@ -55,6 +55,10 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 typedef uint32_t v2u __attribute__((ext_vector_type(2)));
 typedef uint32_t v4u __attribute__((ext_vector_type(4)));
 typedef short v4s __attribute__((ext_vector_type(4)));
+// 16 bytes of `out`, which callers need only align to kOutAlign.
+constexpr int kOutAlign = 8;
+typedef uint32_t v4u_out __attribute__((ext_vector_type(4), aligned(kOutAlign)));
+static_assert(alignof(v4u_out) == kOutAlign && alignof(uint2) <= kOutAlign, "stores of out");
 
 constexpr int kQkDim = 576;
 constexpr int kVDim = 512;
@@ -728,7 +732,7 @@ __global__ __launch_bounds__(kThreads, 1) void sparse_mla_fwd(
         const auto hi = __builtin_amdgcn_permlane16_swap(
             pack_bf16(o[t][m][2] * inv_l, o[t][m][3] * inv_l),
             pack_bf16(o[t][m + 1][2] * inv_l, o[t][m + 1][3] * inv_l), false, false);
-        *reinterpret_cast<uint4*>(orow + 16 * m) = make_uint4(lo[0], hi[0], lo[1], hi[1]);
+        *reinterpret_cast<v4u_out*>(orow + 16 * m) = v4u_out{lo[0], hi[0], lo[1], hi[1]};
       }
     }
   };
@@ -1310,7 +1314,7 @@ int check_common(const void* q, int64_t rows, int64_t heads, const int32_t* indi
   DSA_CHECK_ARG(rows < 0x7FFFFFFF, "too many query rows");
   if (rows == 0) return kOk;
   DSA_CHECK_ARG(q && indices && out, "null pointer");
-  DSA_CHECK_ARG(reinterpret_cast<uintptr_t>(q) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 8 == 0,
+  DSA_CHECK_ARG(reinterpret_cast<uintptr_t>(q) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % kOutAlign == 0,
                 "q must be 16-byte and out 8-byte aligned");
   return kOk;
 }

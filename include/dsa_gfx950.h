@@ -408,7 +408,8 @@ int dsa_index_producer_floors_fp8(
  * operators/deepseek_v32/attention/offload/mla.py:12-20.
  * q: bf16 [rows, heads, 576] (heads a multiple of 64); kv: bf16
  * [kv_rows, 576]; indices: int32 [rows, topk], ids outside [0, kv_rows) are
- * padding; out: bf16 [rows, heads, 512]. softmax scale `scale`.
+ * padding; out: bf16 [rows, heads, 512]. softmax scale `scale`. q and kv are
+ * 16-byte aligned, out 8-byte aligned.
  */
 int dsa_sparse_mla_bf16(const void* q, int64_t rows, int64_t heads, const void* kv,
                         int64_t kv_rows, const int32_t* indices, int64_t topk, float scale,
