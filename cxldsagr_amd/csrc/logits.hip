@@ -793,6 +793,20 @@ EmitLayout emit_layout(int64_t rows, int64_t columns, int64_t list_cap) {
   return l;
 }
 
+// The score area and workspace of the candidate calls (rows >= 1, columns in
+// range: after check_logits_args). Every entry point that queues more than
+// one launch calls it before the first, which already writes the workspace.
+int check_emit_buffers(int64_t rows, int64_t columns, int64_t list_cap, const float* scores,
+                       const void* workspace, int64_t workspace_bytes, EmitLayout* layout) {
+  DSA_CHECK_ARG(scores != nullptr, "null pointer");
+  *layout = emit_layout(rows, columns, list_cap);
+  DSA_CHECK_ARG(layout->plan.splits <= kMaxEmitSplits, "too many key splits");
+  DSA_CHECK_ARG(workspace != nullptr && reinterpret_cast<uintptr_t>(workspace) % 256 == 0 &&
+                    workspace_bytes >= layout->bytes,
+                "indexer select workspace too small or misaligned");
+  return kOk;
+}
+
 }  // namespace
 }  // namespace dsa
 
@@ -899,16 +913,13 @@ extern "C" int dsa_indexer_logits_fp8_emit(const void* q, const void* k, const f
                                            float* scores, int64_t list_cap, void* workspace,
                                            int64_t workspace_bytes, hipStream_t stream) {
   using namespace dsa;
-  const int status = check_logits_args(q, k, weights, kscale, starts, ends, query_start, rows,
-                                       columns, ldo, q_fold);
+  int status = check_logits_args(q, k, weights, kscale, starts, ends, query_start, rows, columns,
+                                 ldo, q_fold);
   if (status != kOk || rows == 0) return status;
   DSA_CHECK_ARG(ldo == (columns + 255) / 256 * 256, "the score stride must be columns rounded up to 256");
-  DSA_CHECK_ARG(scores != nullptr, "null pointer");
-  const EmitLayout l = emit_layout(rows, columns, list_cap);
-  DSA_CHECK_ARG(l.plan.splits <= kMaxEmitSplits, "too many key splits");
-  DSA_CHECK_ARG(workspace != nullptr && reinterpret_cast<uintptr_t>(workspace) % 256 == 0 &&
-                    workspace_bytes >= l.bytes,
-                "indexer select workspace too small or misaligned");
+  EmitLayout l;
+  status = check_emit_buffers(rows, columns, list_cap, scores, workspace, workspace_bytes, &l);
+  if (status != kOk) return status;
   uint8_t* base = static_cast<uint8_t*>(workspace);
   EmitArgs emit{reinterpret_cast<const uint32_t*>(base),
                 reinterpret_cast<uint64_t*>(base + l.lists_offset),
@@ -932,16 +943,14 @@ extern "C" int dsa_indexer_emit_topk(const void* q, const void* k, const float* 
                                      int64_t workspace_bytes, hipStream_t stream) {
   using namespace dsa;
   DSA_CHECK_ARG(topk >= 1 && topk <= 2048, "k must be an integer in [1, 2048]");
-  const int status = check_logits_args(q, k, weights, kscale, starts, ends, query_start, rows,
-                                       columns, columns, q_fold);
+  int status = check_logits_args(q, k, weights, kscale, starts, ends, query_start, rows, columns,
+                                 columns, q_fold);
   if (status != kOk || rows == 0) return status;
   DSA_CHECK_ARG(out_ld >= (topk < columns ? topk : columns), "output row stride too small");
-  DSA_CHECK_ARG(values && indices && scores, "null pointer");
-  const EmitLayout l = emit_layout(rows, columns, list_cap);
-  DSA_CHECK_ARG(l.plan.splits <= kMaxEmitSplits, "too many key splits");
-  DSA_CHECK_ARG(workspace != nullptr && reinterpret_cast<uintptr_t>(workspace) % 256 == 0 &&
-                    workspace_bytes >= l.bytes,
-                "indexer select workspace too small or misaligned");
+  DSA_CHECK_ARG(values && indices, "null pointer");
+  EmitLayout l;
+  status = check_emit_buffers(rows, columns, list_cap, scores, workspace, workspace_bytes, &l);
+  if (status != kOk) return status;
   const uint8_t* base = static_cast<const uint8_t*>(workspace);
   return topk_from_candidates(
       static_cast<const uint8_t*>(q), static_cast<const uint8_t*>(k), weights, kscale, starts,
@@ -1012,7 +1021,9 @@ extern "C" int dsa_layer_indexer_fp8(const void* q, int64_t rows, const float* w
                                      int64_t scratch_bytes, void* workspace,
                                      int64_t workspace_bytes, hipStream_t stream) {
   using namespace dsa;
-  DSA_CHECK_ARG(rows >= 1 && position >= 0 && topk >= 1 && topk <= 2048, "invalid layer indexer shape");
+  DSA_CHECK_ARG(rows >= 1 && rows < 0x7FFFFFFF && position >= 0 && position < 0x7FFFFFFF &&
+                    topk >= 1 && topk <= 2048,
+                "invalid layer indexer shape");
   DSA_CHECK_ARG(index_keys && index_scales && indices, "null pointer");
   const int64_t columns = position + rows;
   const int64_t count = topk < columns ? topk : columns;
@@ -1023,13 +1034,22 @@ extern "C" int dsa_layer_indexer_fp8(const void* q, int64_t rows, const float* w
   uint8_t* base = static_cast<uint8_t*>(scratch);
   float* folded = reinterpret_cast<float*>(base + at.folded);
   float* q_fold = reinterpret_cast<float*>(base + at.fold);
-  int status = dsa_layer_prologue_floors_fp8(
+  const int64_t ldo = (columns + 255) / 256 * 256;
+  // Everything the three launches check, before the first of them: it writes
+  // the floors into the workspace and the new rows into the caches. (The
+  // prologue checks its own arguments ahead of its launch.)
+  int status = check_logits_args(base, index_keys, folded, index_scales, nullptr, nullptr, position,
+                                 rows, columns, ldo, q_fold);
+  if (status != kOk) return status;
+  EmitLayout l;
+  status = check_emit_buffers(rows, columns, 0, scores, workspace, workspace_bytes, &l);
+  if (status != kOk) return status;
+  status = dsa_layer_prologue_floors_fp8(
       q, rows * kHeads, weights, base, reinterpret_cast<float*>(base + at.scales), folded, q_fold, k,
       rows, static_cast<uint8_t*>(index_keys) + position * kDim, index_scales + position, kv,
       kv ? rows : 0, kv ? position : 0, page_table, kv ? pages : 0, cache, nullptr, index_keys,
       index_scales, position, topk, static_cast<uint32_t*>(workspace), stream);
   if (status != kOk) return status;
-  const int64_t ldo = (columns + 255) / 256 * 256;
   status = dsa_indexer_logits_fp8_emit(base, index_keys, folded, index_scales, nullptr, nullptr,
                                        position, rows, columns, ldo, q_fold, scores, 0, workspace,
                                        workspace_bytes, stream);
