@@ -970,10 +970,19 @@ extern "C" int dsa_indexer_select_fp8(const void* q, const void* k, const float*
                                       int64_t out_ld, void* workspace, int64_t workspace_bytes,
                                       hipStream_t stream) {
   using namespace dsa;
-  int status = dsa_indexer_floors_fp8(q, k, weights, kscale, starts, ends, query_start, rows,
-                                      columns, topk, static_cast<uint32_t*>(workspace), stream);
-  if (status != kOk || rows == 0) return status;
+  DSA_CHECK_ARG(topk >= 1 && topk <= 2048, "k must be an integer in [1, 2048]");
   const int64_t ldo = (columns + 255) / 256 * 256;
+  int status = check_logits_args(q, k, weights, kscale, starts, ends, query_start, rows, columns,
+                                 ldo, q_fold);
+  if (status != kOk || rows == 0) return status;
+  DSA_CHECK_ARG(out_ld >= (topk < columns ? topk : columns), "output row stride too small");
+  DSA_CHECK_ARG(values && indices, "null pointer");
+  EmitLayout l;
+  status = check_emit_buffers(rows, columns, 0, scores, workspace, workspace_bytes, &l);
+  if (status != kOk) return status;
+  status = dsa_indexer_floors_fp8(q, k, weights, kscale, starts, ends, query_start, rows, columns,
+                                  topk, static_cast<uint32_t*>(workspace), stream);
+  if (status != kOk) return status;
   status = dsa_indexer_logits_fp8_emit(q, k, weights, kscale, starts, ends, query_start, rows,
                                        columns, ldo, q_fold, scores, 0, workspace, workspace_bytes,
                                        stream);

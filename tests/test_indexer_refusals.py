@@ -36,8 +36,30 @@ def _layer_args(address, stream):
     }
 
 
-def _refused(args):
+def _select_args(address, stream):
+    """The same for dsa_indexer_select_fp8."""
+    workspace = _size("dsa_indexer_select_workspace_bytes", ROWS, COLUMNS, 0)
+    return {
+        "q": address("q", ROWS * 64 * 128), "k": address("k", COLUMNS * 128),
+        "weights": address("weights", ROWS * 256), "kscale": address("kscale", COLUMNS * 4),
+        "starts": None, "ends": None, "query_start": POSITION, "rows": ROWS, "columns": COLUMNS,
+        "q_fold": address("q_fold", ROWS * 2048), "scores": address("scores", ROWS * 512 * 4),
+        "topk": TOPK, "values": address("values", ROWS * TOPK * 4),
+        "indices": address("indices", ROWS * TOPK * 4), "out_ld": TOPK,
+        "workspace": address("workspace", workspace), "workspace_bytes": workspace, "stream": stream,
+    }
+
+
+def _refused(name, args):
     """Variants of valid arguments that the call must refuse."""
+    if name == "dsa_indexer_select_fp8":
+        return [
+            {"workspace_bytes": args["workspace_bytes"] - 1}, {"workspace_bytes": 0},
+            {"workspace": None}, {"workspace": args["workspace"] + 16}, {"scores": None},
+            {"indices": None}, {"values": None}, {"out_ld": TOPK - 1}, {"topk": 0}, {"topk": 2049},
+            {"q": None}, {"q_fold": args["q_fold"] + 4}, {"query_start": POSITION + 1},
+            {"ends": args["kscale"]}, {"columns": 2**26},
+        ]
     return [
         {"workspace_bytes": args["workspace_bytes"] - 1}, {"workspace_bytes": 0},
         {"workspace": None}, {"workspace": args["workspace"] + 16}, {"scores": None},
@@ -48,30 +70,35 @@ def _refused(args):
     ]
 
 
-def _refuses(args, change):
+CALLS = {"dsa_layer_indexer_fp8": _layer_args, "dsa_indexer_select_fp8": _select_args}
+
+
+def _refuses(name, args, change):
     with pytest.raises(ValueError):
-        _native.call("dsa_layer_indexer_fp8", *{**args, **change}.values())
+        _native.call(name, *{**args, **change}.values())
 
 
+@pytest.mark.parametrize("name", CALLS)
 @pytest.mark.skipif(torch.cuda.is_available(), reason="addresses that no device may see")
-def test_layer_indexer_refuses_before_any_launch():
+def test_calls_refuse_before_any_launch(name):
     """Without a device a launch is an error of another kind."""
-    args = _layer_args(lambda name, size: 1 << 20, None)
-    for change in _refused(args):
-        _refuses(args, change)
+    args = CALLS[name](lambda buffer, size: 1 << 20, None)
+    for change in _refused(name, args):
+        _refuses(name, args, change)
 
 
 @pytest.mark.gpu
-def test_refused_layer_calls_write_nothing(gpu):
+@pytest.mark.parametrize("name", CALLS)
+def test_refused_calls_write_nothing(gpu, name):
     buffers = {}
 
-    def address(name, size):
-        buffers[name] = torch.full((size + 256,), 0x5A, dtype=torch.uint8, device=gpu)
-        return buffers[name].data_ptr()
+    def address(buffer, size):
+        buffers[buffer] = torch.full((size + 256,), 0x5A, dtype=torch.uint8, device=gpu)
+        return buffers[buffer].data_ptr()
 
-    args = _layer_args(address, _native.stream_of(gpu))
-    for change in _refused(args):
-        _refuses(args, change)
+    args = CALLS[name](address, _native.stream_of(gpu))
+    for change in _refused(name, args):
+        _refuses(name, args, change)
     torch.cuda.synchronize()
-    for name, buffer in buffers.items():
-        assert bool((buffer == 0x5A).all()), name
+    for buffer, content in buffers.items():
+        assert bool((content == 0x5A).all()), buffer
