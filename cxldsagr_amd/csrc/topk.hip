@@ -1236,26 +1236,30 @@ __device__ __forceinline__ bool counting_sort_buckets(FinishSort& fs, const uint
   return false;
 }
 
-// Linear buckets of the values between the radix keys `lo` and `hi` (finite):
-// false when their span or its reciprocal overflows. The steps round, but
-// none of them can order two values the wrong way.
+__device__ __forceinline__ bool finite_key(uint32_t radix) {
+  return (key_bits(radix) & 0x7F800000u) != 0x7F800000u;
+}
+
+// Linear buckets of the values between the radix keys `lo` and `hi`: false
+// when one is not finite or their span or its reciprocal overflows. The steps
+// round, but none of them can order two values the wrong way. (The bits decide
+// what is finite, ahead of any arithmetic: this file is compiled to assume no
+// NaN in a float operation, whose result would then be anything.)
 struct ValueBuckets {
-  float least, per;
+  float least = 0.0f, per = 0.0f;
   __device__ __forceinline__ bool set(uint32_t lo, uint32_t hi) {
+    if (!finite_key(lo) || !finite_key(hi)) return false;
     least = __uint_as_float(key_bits(lo));
     const float span = __uint_as_float(key_bits(hi)) - least;
+    if (!(span == 0.0f || (span >= 1e-30f && span <= 1e37f))) return false;
     per = span > 0.0f ? (float)(kSortBins - 1) / span : 0.0f;
-    return span <= 1e37f && (span == 0.0f || span >= 1e-30f);
+    return true;
   }
   __device__ __forceinline__ uint32_t operator()(uint64_t k) const {
     const float x = (__uint_as_float(key_bits((uint32_t)(k >> 32))) - least) * per;
     return min((uint32_t)fmaxf(x, 0.0f), (uint32_t)kSortBins - 1);
   }
 };
-
-__device__ __forceinline__ bool finite_key(uint32_t radix) {
-  return (key_bits(radix) & 0x7F800000u) != 0x7F800000u;
-}
 
 // The same for keys whose radix keys lie in [lo, hi]: buckets of the values,
 // or, where an end is not finite or the span extreme, of the radix keys.
@@ -1273,7 +1277,7 @@ __device__ __forceinline__ bool counting_sort_mask(FinishSort& fs, const uint64_
   const int bits = 32 - __builtin_clz((span - 1) | 1u);
   const int shift = bits > 12 ? bits - 12 : 0;
   ValueBuckets of_value;
-  const bool by_value = of_value.set(lo, hi) && finite_key(lo) && finite_key(hi);
+  const bool by_value = of_value.set(lo, hi);
   auto bucket_of = [=](uint64_t k) -> uint32_t {
     if (by_value) return of_value(k);
     return min(((uint32_t)(k >> 32) - lo) >> shift, (uint32_t)kSortBins - 1);
