@@ -1240,46 +1240,91 @@ __device__ __forceinline__ bool finite_key(uint32_t radix) {
   return (key_bits(radix) & 0x7F800000u) != 0x7F800000u;
 }
 
-// Linear buckets of the values between the radix keys `lo` and `hi`: false
-// when one is not finite or their span or its reciprocal overflows. The steps
-// round, but none of them can order two values the wrong way. (The bits decide
+// The values between the radix keys `lo` and `hi`, for buckets: false when one
+// is not finite or their span or its reciprocal overflows. (The bits decide
 // what is finite, ahead of any arithmetic: this file is compiled to assume no
-// NaN in a float operation, whose result would then be anything.)
-struct ValueBuckets {
-  float least = 0.0f, per = 0.0f;
+// NaN in a float operation, whose result would then be anything.) The steps of
+// both kinds of buckets round, but none of them can order two values the
+// wrong way. Every value must lie in the range (one outside it, as counts that
+// disagree with the scores can give, indexes no other memory).
+struct ValueRange {
+  float least = 0.0f, span = 0.0f;
   __device__ __forceinline__ bool set(uint32_t lo, uint32_t hi) {
     if (!finite_key(lo) || !finite_key(hi)) return false;
     least = __uint_as_float(key_bits(lo));
-    const float span = __uint_as_float(key_bits(hi)) - least;
-    if (!(span == 0.0f || (span >= 1e-30f && span <= 1e37f))) return false;
-    per = span > 0.0f ? (float)(kSortBins - 1) / span : 0.0f;
-    return true;
+    span = __uint_as_float(key_bits(hi)) - least;
+    return span == 0.0f || (span >= 1e-30f && span <= 1e37f);
+  }
+  __device__ __forceinline__ float above(uint64_t k) const {
+    return fmaxf(__uint_as_float(key_bits((uint32_t)(k >> 32))) - least, 0.0f);
+  }
+};
+// Buckets of equal width: for the whole of a row, whose ends hold few values.
+struct LinearBuckets {
+  ValueRange range;
+  float per;
+  __device__ __forceinline__ explicit LinearBuckets(const ValueRange& r)
+      : range(r), per(r.span > 0.0f ? (float)(kSortBins - 1) / r.span : 0.0f) {}
+  __device__ __forceinline__ uint32_t operator()(uint64_t k) const {
+    return min((uint32_t)(range.above(k) * per), (uint32_t)kSortBins - 1);
+  }
+};
+// Buckets of equal ratio of the distance from the range's low end, 256 per
+// octave over the 16 octaves below the span (the first bucket takes the rest):
+// for the values above a threshold, which are densest at it. However far a few
+// of them lie above the others (up to 2^16 times), the others keep their share of
+// the buckets.
+struct DistanceBuckets {
+  ValueRange range;
+  static constexpr int kShift = 15;
+  static_assert(kSortBins >> (23 - kShift) == 16, "octaves");
+  __device__ __forceinline__ uint32_t operator()(uint64_t k) const {
+    const uint32_t below = (__float_as_uint(range.span) - __float_as_uint(range.above(k))) >> kShift;
+    return (uint32_t)kSortBins - 1 - min(below, (uint32_t)kSortBins - 1);
+  }
+};
+// The same for a whole row with a few values far from the rest: 128 per octave
+// over the 32 octaves below the span, or, where the range crosses zero, 64 on
+// each side of it.
+struct SpreadBuckets {
+  float centre, reach;
+  int shift;
+  uint32_t side;  // buckets of one side
+  __device__ __forceinline__ explicit SpreadBuckets(const ValueRange& r) {
+    const bool crosses = r.least < 0.0f && r.least + r.span > 0.0f;
+    centre = crosses ? 0.0f : r.least;
+    reach = crosses ? fmaxf(-r.least, r.least + r.span) : r.span;
+    shift = crosses ? 17 : 16;
+    side = crosses ? kSortBins / 2 : kSortBins;
   }
   __device__ __forceinline__ uint32_t operator()(uint64_t k) const {
-    const float x = (__uint_as_float(key_bits((uint32_t)(k >> 32))) - least) * per;
-    return min((uint32_t)fmaxf(x, 0.0f), (uint32_t)kSortBins - 1);
+    const float d = __uint_as_float(key_bits((uint32_t)(k >> 32))) - centre;
+    const float m = fminf(fabsf(d), reach);
+    const uint32_t below = min((__float_as_uint(reach) - __float_as_uint(m)) >> shift, side - 1);
+    return d < 0.0f ? below : (uint32_t)kSortBins - 1 - below;
   }
 };
 
-// The same for keys whose radix keys lie in [lo, hi]: buckets of the values,
-// or, where an end is not finite or the span extreme, of the radix keys.
-// (Radix buckets put most keys of a range that crosses zero - a row whose
-// threshold is negative, as of one in a few hundred at 64K columns, more at
-// fewer - into a few dozen buckets, too crowded to rank, and one such row sets
-// the launch: 128 rows x 65,664 columns 17.7 -> 9.2 us, 37 x 20,048 25.9 -> 9.1.)
-// Keys outside the range only come with counts that disagree with the
-// scores; they are clamped, so that they index no other memory.
+// The same for keys whose radix keys lie in [lo, hi], lo a threshold: buckets
+// by the distance from it, or, where an end is not finite or the span extreme, of
+// the radix keys. One crowded row, which must refine its keys first, sets the
+// launch; 128 rows x 65,664 columns / 37 x 20,048, us:
+//                                              radix        linear       distance
+//   scores around zero (some thresholds negative)  11.7 / 36.3  9.4 / 8.7    9.5 / 8.8
+//   all scores positive                         8.7 / 19.3   9.4 / 8.9    9.5 / 8.8
+//   a few columns 100 times the rest           11.7 / 36.4  30.8 / 20.8  9.5 / 8.8
+//   the same, all positive                     10.0 / 20.4  33.4 / 30.0  9.3 / 8.8
 template <typename Emit>
 __device__ __forceinline__ bool counting_sort_mask(FinishSort& fs, const uint64_t (&key)[kSortPerThread],
                                                    uint32_t valid, uint32_t n, uint32_t lo,
                                                    uint32_t hi, int count, Emit&& emit) {
+  ValueRange range;
+  if (range.set(lo, hi))
+    return counting_sort_buckets(fs, key, valid, n, DistanceBuckets{range}, count, emit);
   const uint32_t span = hi - lo + 1u;  // 0 stands for 2^32
   const int bits = 32 - __builtin_clz((span - 1) | 1u);
   const int shift = bits > 12 ? bits - 12 : 0;
-  ValueBuckets of_value;
-  const bool by_value = of_value.set(lo, hi);
   auto bucket_of = [=](uint64_t k) -> uint32_t {
-    if (by_value) return of_value(k);
     return min(((uint32_t)(k >> 32) - lo) >> shift, (uint32_t)kSortBins - 1);
   };
   return counting_sort_buckets(fs, key, valid, n, bucket_of, count, emit);
@@ -1288,10 +1333,13 @@ __device__ __forceinline__ bool counting_sort_mask(FinishSort& fs, const uint64_
 // The top `count` of a row of which at most kSortCap columns, [lo, hi), are
 // visible (the others are -inf): every finite score goes into one counting
 // sort over kSortBins linear buckets of the values between the row's smallest
-// and largest, then -inf / -1 slots. Returns false, with nothing written, for
-// a row with a NaN, +inf or an extreme span, or a crowded bucket (many
-// near-equal scores). The
-// work-group's threads call it together.
+// and largest, then -inf / -1 slots; where a bucket is crowded, once more over
+// buckets that spread a row with a few scores far from the rest (columns 100
+// times the others: 128 rows x 4,224 columns 30.7 -> 15.3 us, x 8,192 30.4 ->
+// 16.0 against the whole of select_row; 2,048 x 2,048 130 -> 70). Returns false, with
+// nothing written, for a row with a NaN, +inf or an extreme span, or a bucket
+// that stays crowded (many near-equal scores). The work-group's threads call it
+// together.
 template <typename Emit>
 __device__ __forceinline__ bool sort_visible(FinishSort& fs, uint4* __restrict__ wave_parts,
                                              const float* __restrict__ row, int64_t lo, int64_t hi,
@@ -1354,9 +1402,15 @@ __device__ __forceinline__ bool sort_visible(FinishSort& fs, uint4* __restrict__
   if (odd) return false;
   const int found = n < (uint32_t)count ? (int)n : count;
   if (found > 0) {
-    ValueBuckets bucket_of;
-    if (!bucket_of.set(smallest, largest)) return false;
-    if (!counting_sort_buckets(fs, key, valid, n, bucket_of, found, emit)) return false;
+    ValueRange range;
+    if (!range.set(smallest, largest) || (range.span == 0.0f && n > kSortBucketMax)) return false;
+    if (!counting_sort_buckets(fs, key, valid, n, LinearBuckets(range), found, emit)) {
+      __syncthreads();
+      for (int i = tid; i < kSortBins; i += kThreads) fs.cursor[i] = 0;
+      if (tid == 0) fs.crowded = 0;
+      __syncthreads();
+      if (!counting_sort_buckets(fs, key, valid, n, SpreadBuckets(range), found, emit)) return false;
+    }
   }
   for (int i = found + tid; i < count; i += kThreads) emit(i, (uint64_t)0x007FFFFFu << 32);
   return true;
@@ -1815,7 +1869,13 @@ __global__ __launch_bounds__(kThreads, 1) void topk_candidates(float* __restrict
 #pragma unroll
     for (int j = 0; j < kSortPerThread; ++j)
       key[j] = (valid >> j) & 1u ? fs.sorted[tid + j * kThreads] : 0ull;
+    // The largest key of all lists (top_all has those that fit the registers).
+    uint32_t most = 0;
+#pragma unroll
+    for (int j = 0; j < kSortPerThread; ++j) most = max(most, (uint32_t)(key[j] >> 32));
+    atomicMax(&info[1], most);
     __syncthreads();  // the sort scatters into the buffer
+    top_all = info[1];
   }
   // Fewer than `count` candidates: the floor was above the count-th
   // largest score, and scores below it are missing.
