@@ -1208,36 +1208,46 @@ __global__ __launch_bounds__(kValueThreads, kDv < 256 ? 2 : 1) void mla_values(
 // How a call's rows are run: rows [0, wide_rows) by sparse_mla_fwd, the rest in
 // the split form with kDv = dv.
 //
-// sparse_mla_fwd takes about 76 us (2,048 selected) for each round of one
-// (row, 64 heads) work-group per CU, however few there are. The split form,
-// whose scores go through memory instead of LDS, measured 35 / 43 / 54 / 77 us
-// for 4 / 16 / 32 / 64 rows of 128 heads over 2,048 fp8 records (56 / 92 us
-// for 32 / 64 rows of bf16 records), so the rows after the last full round go
-// there while they are at most a quarter of a round. It also wants some
-// length to spread: at 500 selected 19.7 us against 26.4, at 33 20.0 against
-// 17.6.
+// sparse_mla_fwd takes about 71 us (2,048 selected; 40 us at 1,024, 24 at 512, 18
+// at 320) for each round of one (row, 64 heads) work-group per CU, however few
+// there are. The split form's scores go through memory instead of LDS, so the
+// rows after the last full round go there while they are few enough. Rows of
+// 128 heads over fp8 / bf16 records, us, the split form beside the wide one:
+//   2,048 selected  4 rows 34 / 32 (71)  16 rows 43 / 40 (72)  32 rows 54 / 56 (72)
+//                   36 rows 78 / 88 (71 / 73)  64 rows 83 / 100 (73)
+// so never above a quarter of a round. Below it needs some length to spread,
+// the more the fuller the round (`least`); at the lines it is the faster form:
+//   up to a sixteenth  320 selected  1 row 18.2 / 17.2 (17.7 / 17.3)  4 rows 18.4 / 17.0 (18.2 / 17.8)
+//   up to an eighth    448           16 rows 21.4 / 20.4 (22.3 / 22.0); at 320 21.8 / 20.0 (18.2 / 17.9)
+//   up to a quarter    20 rows 640   28.1 / 28.0 (28.4 / 28.2); at 512 24.3 / 24.1 (24.2)
+//                      32 rows 784   about 33 (32.5); at 640 32.2 / 32.9 (28.5), at 1,024 37.2 / 37.1 (40)
+// (mla_scores deals a run of key blocks to each work-group, and a run length
+// that leaves a few work-groups to a second round is slower than the wide form all
+// the same: 24 rows x 1,024 selected 41.8 / 41.2 against 39.8 / 40.5.)
 struct MlaPlan {
   int64_t wide_rows, split_rows;
   int dv;
   int64_t score_floats, bytes;  // of the split rows' workspace: scores, then block maxima
 };
 
-constexpr int64_t kSplitMinSelected = 320;
-
 MlaPlan mla_plan(int64_t rows, int64_t heads, int64_t topk) {
   MlaPlan p{rows, 0, 0, 0, 0};
   const int64_t cus = device_cu_count();
   const int64_t per_row = heads / kHeadsPerGroup;
-  if (topk < kSplitMinSelected || topk > kSplitSelected || per_row * 4 > cus) return p;
+  if (topk > kSplitSelected || per_row * 4 > cus) return p;
   const int64_t round = cus / per_row;  // rows of a full round
   const int64_t tail = rows % round;
-  if (tail == 0 || tail * per_row * 4 > cus) return p;
+  const int64_t tiles = tail * per_row;
+  if (tail == 0 || tiles * 4 > cus) return p;
+  const int64_t least = tiles * 16 <= cus ? 320 : tiles * 8 <= cus ? 448 : 384 + 1600 * tiles / cus;
+  if (topk < least) return p;
   p.wide_rows = rows - tail;
   p.split_rows = tail;
   // One round of mla_values work-groups at 64 dims up to an eighth of the
-  // CUs' tiles; above, 128 dims halve the softmax work (each part of the
-  // dims repeats it).
-  p.dv = tail * per_row * 8 <= cus ? 64 : 128;
+  // CUs' tiles; above, 128 dims halve the softmax work, which each part of the
+  // dims repeats (2,048 selected: 16 rows of 128 heads 42.9 / 40.4 us with 64 dims and 47.0 / 46.1
+  // with 128, 20 rows 61.4 / 57.4 and 58.1 / 56.6).
+  p.dv = tiles * 8 <= cus ? 64 : 128;
   p.score_floats = tail * padded_blocks(topk) * heads * kBlock;
   p.bytes = (p.score_floats + tail * padded_blocks(topk) * heads) * 4;
   return p;
