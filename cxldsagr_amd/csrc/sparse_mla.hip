@@ -1221,9 +1221,6 @@ __global__ __launch_bounds__(kValueThreads, kDv < 256 ? 2 : 1) void mla_values(
 //   up to an eighth    448           16 rows 21.4 / 20.4 (22.3 / 22.0); at 320 21.8 / 20.0 (18.2 / 17.9)
 //   up to a quarter    20 rows 640   28.1 / 28.0 (28.4 / 28.2); at 512 24.3 / 24.1 (24.2)
 //                      32 rows 784   about 33 (32.5); at 640 32.2 / 32.9 (28.5), at 1,024 37.2 / 37.1 (40)
-// (mla_scores deals a run of key blocks to each work-group, and a run length
-// that leaves a few work-groups to a second round is slower than the wide form all
-// the same: 24 rows x 1,024 selected 41.8 / 41.2 against 39.8 / 40.5.)
 struct MlaPlan {
   int64_t wide_rows, split_rows;
   int dv;
@@ -1260,12 +1257,15 @@ int launch_split(const MlaPlan& p, const uint16_t* q, int64_t heads, const uint8
   const int64_t rows = p.split_rows;
   float* block_max = scores + p.score_floats;
   // mla_scores: all heads of a multiple of 128 share a staged block, and the
-  // blocks are dealt out for about one work-group per CU.
+  // blocks are dealt out for at most one work-group per CU: runs a step shorter
+  // than that leave a few work-groups to a second round (12 rows of 128 heads,
+  // 2,048 selected, 47.7 us as 264 work-groups, 39.8 as 192; 24 rows 59.7, 50.9).
   const int tiles = heads % 128 == 0 ? 4 : 2;
   const int64_t steps = padded_blocks(topk) * tiles / 4;
   const int64_t units = rows * (heads / (32 * tiles));
   const int64_t most = kScoreKeys / kBlock * tiles / 4;
-  int64_t chunk = (units * steps + device_cu_count() - 1) / device_cu_count();
+  const int64_t fit = device_cu_count() / units;  // runs per unit in one round
+  int64_t chunk = (steps + (fit > 1 ? fit : 1) - 1) / (fit > 1 ? fit : 1);
   if (chunk > most) chunk = most;
   const int64_t chunks = (steps + chunk - 1) / chunk;
   hipLaunchKernelGGL((tiles == 4 ? mla_scores<kFp8, 4> : mla_scores<kFp8, 2>),

@@ -108,3 +108,33 @@ def test_rows_that_end_in_padding_equal_their_short_selections(gpu, heads):
         want = (sparse_mla(q[r:r + 1], kv, ids[r:r + 1, :end].contiguous(), SCALE)[0] if end
                 else torch.zeros_like(got[r]))
         assert torch.equal(got[r].view(torch.int16), want.view(torch.int16)), end
+
+
+@pytest.mark.parametrize("fewer,more,heads,selected", [(12, 16, 128, 2048), (26, 32, 128, 2048),
+                                                       (24, 32, 128, 1024), (24, 32, 64, 2048)])
+def test_fewer_rows_take_no_longer(gpu, fewer, more, heads, selected):
+    """The score launch's runs fit one round of work-groups for every row count
+    (fewer rows had taken 1.10 to 1.13 times as long as more)."""
+    from cxldsagr_amd.attention import sparse_mla
+
+    gen = torch.Generator(device=gpu).manual_seed(1)
+    kv = torch.randn(20000, 576, generator=gen, device=gpu).bfloat16()
+
+    def call(rows):
+        q = torch.randn(rows, heads, 576, generator=gen, device=gpu).bfloat16()
+        ids = torch.randint(0, 20000, (rows, selected), generator=gen, device=gpu).int()
+        return lambda: sparse_mla(q, kv, ids, SCALE)
+
+    calls, best = [call(fewer), call(more)], [float("inf")] * 2
+    for fn in calls:
+        fn()
+    for _ in range(9):
+        for i, fn in enumerate(calls):
+            begin, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            begin.record()
+            for _ in range(30):
+                fn()
+            end.record()
+            torch.cuda.synchronize()
+            best[i] = min(best[i], begin.elapsed_time(end))
+    assert best[0] < 1.04 * best[1], best
