@@ -1215,17 +1215,20 @@ __global__ __launch_bounds__(kValueThreads, kDv < 256 ? 2 : 1) void mla_values(
 // 128 heads over fp8 / bf16 records, us, the split form beside the wide one:
 //   2,048 selected  4 rows 34 / 32 (71)  16 rows 43 / 40 (72)  32 rows 54 / 56 (72)
 //                   36 rows 78 / 88 (71 / 73)  64 rows 83 / 100 (73)
-// so never above a quarter of a round. Below it needs some length to spread,
-// the more the fuller the round (`least`); at the lines it is the faster form:
-//   up to a sixteenth  320 selected  1 row 18.2 / 17.2 (17.7 / 17.3)  4 rows 18.4 / 17.0 (18.2 / 17.8)
-//   up to an eighth    448           16 rows 21.4 / 20.4 (22.3 / 22.0); at 320 21.8 / 20.0 (18.2 / 17.9)
-//   up to a quarter    20 rows 640   28.1 / 28.0 (28.4 / 28.2); at 512 24.3 / 24.1 (24.2)
-//                      32 rows 784   about 33 (32.5); at 640 32.2 / 32.9 (28.5), at 1,024 37.2 / 37.1 (40)
+// so never above a quarter of a round. Below it the form of less time goes, by
+// costs fitted to both (us; 17 selections of 256 .. 2,048, 33 counts of rows of 64, 128 and
+// 192 heads, both formats; the form taken is within 5 % of the faster one in
+// each): the wide form by its 64-key steps, the split form by its tiles (row, 64
+// heads) and 256-key rounds. At 320 selected 16 rows take 18.2 / 17.9 wide (split 21.8 /
+// 20.0), at 512 24.4 / 24.0 (21.9 / 20.9), 32 rows at 768 32.1 / 32.6 (32.7 / 33.2), at 1,024
+// 39.9 / 40.4 (37.2 / 37.1). Below 320 selected the split form gains at most 1 us.
 struct MlaPlan {
   int64_t wide_rows, split_rows;
   int dv;
   int64_t score_floats, bytes;  // of the split rows' workspace: scores, then block maxima
 };
+
+constexpr int64_t kSplitMinSelected = 320;
 
 MlaPlan mla_plan(int64_t rows, int64_t heads, int64_t topk) {
   MlaPlan p{rows, 0, 0, 0, 0};
@@ -1236,8 +1239,11 @@ MlaPlan mla_plan(int64_t rows, int64_t heads, int64_t topk) {
   const int64_t tail = rows % round;
   const int64_t tiles = tail * per_row;
   if (tail == 0 || tiles * 4 > cus) return p;
-  const int64_t least = tiles * 16 <= cus ? 320 : tiles * 8 <= cus ? 448 : 384 + 1600 * tiles / cus;
-  if (topk < least) return p;
+  const double t = (double)tiles, steps = (double)((topk + 63) / 64), rounds = (double)((topk + 255) / 256);
+  const double wide_us = 8.9 + 1.98 * steps;
+  const double split_us = tiles * 8 <= cus ? 12.5 + 0.049 * t + (2.28 + 0.0453 * t) * rounds
+                                           : 12.8 + 0.065 * t + (3.39 + 0.0304 * t) * rounds;
+  if (topk < kSplitMinSelected || split_us >= wide_us) return p;
   p.wide_rows = rows - tail;
   p.split_rows = tail;
   // One round of mla_values work-groups at 64 dims up to an eighth of the

@@ -33,9 +33,9 @@ def _one_launch(q, cache, table, kv, ids, n_tokens, scale):
     (1, 128, 2048), (1, 64, 321), (2, 192, 1000), (16, 128, 2047), (17, 128, 545),
     (32, 128, 2048), (33, 128, 700), (64, 64, 1025), (65, 64, 320), (129, 128, 640),
     (160, 128, 351), (161, 128, 352), (3, 128, 319), (3, 128, 2049), (5, 64, 511),
-    # Both sides of the shortest selection, which grows with the rows.
-    (8, 128, 320), (9, 128, 447), (9, 128, 448), (17, 128, 595), (17, 128, 596), (32, 128, 783),
-    (160, 128, 784), (64, 64, 784), (21, 192, 777), (10, 192, 448),
+    # Both sides of the selections at which it begins to be the faster form.
+    (8, 128, 320), (9, 128, 320), (9, 128, 321), (16, 128, 384), (16, 128, 385), (17, 128, 448),
+    (17, 128, 449), (17, 128, 513), (32, 128, 960), (160, 128, 961), (64, 64, 962), (21, 192, 1000),
 ])
 def test_split_form_has_the_bits_of_one_launch(gpu, rows, heads, selected):
     from cxldsagr_amd.attention import pack_kv_fp8, sparse_mla, sparse_mla_fp8_paged

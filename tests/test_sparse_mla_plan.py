@@ -21,7 +21,9 @@ def _needs_workspace(rows, heads, selected):
     (4, 128, 2048, 34.3, 71.2), (16, 128, 2048, 42.9, 71.9), (32, 128, 2048, 54.2, 71.6),
     (64, 64, 2048, 58.7, 72.6), (16, 128, 448, 21.4, 22.3), (4, 128, 384, 18.6, 20.2),
     (20, 128, 768, 28.3, 32.1), (28, 128, 1024, 35.2, 40.0), (32, 128, 1024, 37.2, 39.9),
-    (10, 192, 512, 22.7, 24.2), (128 + 16, 128, 448, 21.4, 22.3),
+    (10, 192, 512, 22.7, 24.2), (128 + 16, 128, 448, 21.4, 22.3), (28, 128, 832, 36.4, 34.0),
+    (32, 128, 832, 38.0, 34.0), (64, 64, 832, 38.5, 34.3), (21, 192, 832, 37.7, 34.2),
+    (32, 128, 896, 38.1, 36.0), (24, 128, 704, 29.6, 30.2), (24, 128, 1024, 34.4, 39.8),
 ])
 def test_the_faster_form_is_taken(rows, heads, selected, split, wide):
     if _native.torch.cuda.is_available():
