@@ -1873,7 +1873,13 @@ __global__ __launch_bounds__(kThreads, 1) void topk_candidates(float* __restrict
     uint32_t most = 0;
 #pragma unroll
     for (int j = 0; j < kSortPerThread; ++j) most = max(most, (uint32_t)(key[j] >> 32));
-    atomicMax(&info[1], most);
+    most = max(most, lane_xor<1>(most));
+    most = max(most, lane_xor<2>(most));
+    most = max(most, lane_xor<4>(most));
+    most = max(most, lane_xor<8>(most));
+    most = max(most, lane_xor<16>(most));
+    most = max(most, lane_xor<32>(most));
+    if (lane == 0) atomicMax(&info[1], most);
     __syncthreads();  // the sort scatters into the buffer
     top_all = info[1];
   }
