@@ -45,6 +45,7 @@
 // is written as a composite top-k key into the row's list for the split, and
 // the score matrix is not written (see logits_fp8_mfma's kModeEmit notes).
 #include "logits_core.h"
+#include "logits_plan.h"
 #include "../../include/dsa_gfx950.h"
 
 namespace dsa {
@@ -160,7 +161,7 @@ __global__ __launch_bounds__(kThreads, 1) void logits_fp8_mfma(
     const float* __restrict__ kscale, const int32_t* __restrict__ starts,
     const int32_t* __restrict__ ends, int64_t query_start, int64_t rows, int64_t columns,
     int64_t ldo, int64_t keys_per_split, const float* __restrict__ q_fold, float* __restrict__ out,
-    uint32_t* __restrict__ digit_counts, EmitArgs emit, uint32_t qgroups) {
+    uint32_t* __restrict__ digit_counts, EmitArgs emit, uint32_t qgroups, uint32_t live_splits) {
   constexpr bool kCount = kMode == kModeCount;
   constexpr bool kEmit = kMode == kModeEmit;
   __shared__ __align__(16) uint8_t ring[kRing][kStageBytes];
@@ -178,13 +179,9 @@ __global__ __launch_bounds__(kThreads, 1) void logits_fp8_mfma(
   const int lane = tid & 63;
   const int group = lane >> 4;
   const int col = lane & 15;
-  // Work-groups go to the XCDs round-robin by linear id: XCD e takes the e-th
-  // eighth of the (key split, query group) pairs in split order, so each XCD
-  // gets as many pairs as the others and the query groups of a key range
-  // share its keys through one XCD's L2.
-  const uint32_t pair = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
-  const uint32_t split = pair / qgroups;
-  const int64_t q0 = (int64_t)(pair % qgroups) * kQueriesPerBlock;
+  const SplitPair pair = dealt_pair(blockIdx.x, qgroups, live_splits);
+  const uint32_t split = pair.split;
+  const int64_t q0 = (int64_t)pair.group * kQueriesPerBlock;
   const int64_t kb = (int64_t)split * keys_per_split;
   if (kb >= ldo) return;  // past the last pair (whole work-group, before any barrier)
   const int64_t ke = kb + keys_per_split < ldo ? kb + keys_per_split : ldo;
@@ -680,44 +677,10 @@ __global__ __launch_bounds__(kFloorThreads) void index_floors(
 namespace dsa {
 namespace {
 
-// Key range per work-group. `splits` is the stride of the per-split output
-// (a multiple of 8 from 8 on); `live` of them hold keys and are launched, for
-// each query group.
-struct SplitPlan {
-  int64_t qgroups, splits, per, live;
-  unsigned grid() const { return (unsigned)((live * qgroups + 7) / 8 * 8); }
-};
-
-// The split with the least time by rounds of one work-group per CU, each
-// kStartUs (operands and first keys) plus kStageUs per 128 keys (the stage's
-// MFMAs; both measured). Splitting for at least one work-group per CU and
-// padding the splits to a multiple of 8 left a few work-groups, or one XCD's,
-// to a second round that took as long as the first: 100 rows x 50,001 keys
-// 81.8 -> 48.0 us, 200 rows x 16,584 keys 59.8 -> 34.6 us.
-constexpr double kStartUs = 8.0, kStageUs = 3.0;
-
+// `counted`: the 16-bit LDS digit counters bound a split's keys.
 SplitPlan split_plan(int64_t rows, int64_t ldo, bool counted) {
-  SplitPlan p;
-  p.qgroups = (rows + kQueriesPerBlock - 1) / kQueriesPerBlock;
-  const int64_t cus = device_cu_count();
-  const int64_t stages = (ldo + kStageKeys - 1) / kStageKeys;
-  const int64_t most = stages < cus ? stages : cus;
-  double best = 0.0;
-  p.per = stages * kStageKeys;
-  for (int64_t s = 1; s <= most; ++s) {
-    const int64_t per_stages = (stages + s - 1) / s;
-    const int64_t live = (stages + per_stages - 1) / per_stages;
-    const int64_t rounds = (live * p.qgroups + cus - 1) / cus;
-    const double cost = (double)rounds * (kStartUs + kStageUs * (double)per_stages);
-    if (s == 1 || cost < best) {
-      best = cost;
-      p.per = per_stages * kStageKeys;
-    }
-  }
-  if (counted && p.per > kMaxSplitKeys) p.per = kMaxSplitKeys;  // 16-bit LDS counters
-  p.live = (ldo + p.per - 1) / p.per;
-  p.splits = p.live >= 8 ? (p.live + 7) / 8 * 8 : p.live;
-  return p;
+  return dsa::split_plan(rows, ldo, kQueriesPerBlock, kStageKeys, counted ? kMaxSplitKeys : 0,
+                         device_cu_count());
 }
 
 int check_logits_args(const void* q, const void* k, const float* weights, const float* kscale,
@@ -756,7 +719,7 @@ int logits_launch(const void* q, const void* k, const float* weights, const floa
                      dim3(p.grid()), dim3(kThreads), 0, stream,
                      static_cast<const uint8_t*>(q), static_cast<const uint8_t*>(k), weights,
                      kscale, starts, ends, query_start, rows, columns, ldo, p.per, q_fold, out,
-                     digit_counts, EmitArgs{}, (uint32_t)p.qgroups);
+                     digit_counts, EmitArgs{}, (uint32_t)p.qgroups, (uint32_t)p.live);
   DSA_CHECK_LAUNCH("indexer logits");
   return kOk;
 }
@@ -929,7 +892,7 @@ extern "C" int dsa_indexer_logits_fp8_emit(const void* q, const void* k, const f
                      dim3(kThreads), 0, stream, static_cast<const uint8_t*>(q),
                      static_cast<const uint8_t*>(k), weights, kscale, starts, ends, query_start,
                      rows, columns, ldo, l.plan.per, q_fold, scores, nullptr, emit,
-                     (uint32_t)l.plan.qgroups);
+                     (uint32_t)l.plan.qgroups, (uint32_t)l.plan.live);
   DSA_CHECK_LAUNCH("indexer logits (candidates)");
   return kOk;
 }
