@@ -2026,7 +2026,11 @@ int topk_from_candidates(const uint8_t* q, const uint8_t* k, const float* weight
   DSA_CHECK_ARG(splits >= 1 && splits <= kMaxCandidateSplits, "too many key splits");
   DSA_CHECK_ARG(columns < (int64_t)0x7FFFFFFF && rows < 0x7FFFFFFF, "too many rows or columns");
   const int64_t count = topk < columns ? topk : columns;
-  hipLaunchKernelGGL((columns <= kSortCap ? topk_candidates<true> : topk_candidates<false>),
+  // A few rows of a few columns: the sort's 4,096 buckets cost more than
+  // select_row does (1 row x 64 columns of the whole call 20.2 against 18.9 us, 16 x 200 22.8 against
+  // 21.7; 1 x 300 20.9 against 20.3 and x 400 21.0 against 24.8, 40 x 64 22.7 against 23.0).
+  const bool tiny = columns <= 200 && rows <= 16;
+  hipLaunchKernelGGL((columns <= kSortCap && !tiny ? topk_candidates<true> : topk_candidates<false>),
                      dim3((unsigned)rows), dim3(kThreads), 0, stream, scores, columns, ld, (int)count, values, indices, out_ld,
                      CandidateLists{floors, records, lists, splits, per, cap},
                      LogitsInputs{q, k, weights, kscale, starts, ends, query_start, q_fold});

@@ -34,7 +34,7 @@ def _check(q8, k8, w, ks, start, topk, bounds=None):
 @pytest.mark.parametrize("rows,columns,topk", [
     (1, 1, 2048), (2, 2, 1), (5, 63, 64), (40, 2047, 2048), (33, 2048, 2048), (33, 2049, 2048),
     (7, 4096, 2048), (300, 5000, 777), (3, 8191, 2048), (3, 8192, 2048), (3, 8193, 2048),
-    (40, 8200, 2048),
+    (40, 8200, 2048), (16, 200, 2048), (16, 201, 2048), (17, 200, 2048), (3, 130, 7),
 ])
 def test_short_rows_equal_unfused(gpu, rows, columns, topk):
     q8, k8, w, ks, _ = _inputs(gpu, rows, columns, columns)
