@@ -142,9 +142,9 @@ STAGES = ("marker", "prologue", "logits", "topk", "sparse_mla")
 def in_layer_stage_us(torch, layer, history, tokens, topk, iters, args):
     """Average duration of each stage of the layer step, from HIP events recorded
     between its launches on the current stream (the same launches, in the same
-    order, as DSALayer.forward; the per-row floors are part of the prologue
-    launch), after an empty bracket that measures what one event marker adds
-    to a stage. Also returns the candidate keys the indexer step listed and
+    order, as DSALayer.forward, which queues the indexer's three in one native
+    call; the per-row floors are part of the prologue launch), after an empty
+    bracket that measures what one event marker adds to a stage. Also returns the candidate keys the indexer step listed and
     the key splits that spilled."""
     index_q, index_k, weights, mla_q, kv = args
     fused = layer._fused_prologue_applies(index_q, index_k, weights, kv)
@@ -155,6 +155,7 @@ def in_layer_stage_us(torch, layer, history, tokens, topk, iters, args):
     workspace = select_workspace(rows, tokens, layer.device)
     floors = workspace[:8 * rows].view(torch.int32).view(rows, 2)
 
+    from cxldsagr_amd import indexer
     from cxldsagr_amd.layer import index_prologue
 
     def prologue():
@@ -185,15 +186,9 @@ def in_layer_stage_us(torch, layer, history, tokens, topk, iters, args):
         ev[5].record(stream)
     torch.cuda.synchronize()
     # Candidates listed per row (records [rows][splits][2] after the floors).
-    records_at = (8 * rows + 255) // 256 * 256
-    width = (tokens + 255) // 256 * 256
-    cus = torch.cuda.get_device_properties(layer.device).multi_processor_count
-    qgroups = (rows + 15) // 16
-    splits = max(1, (cus + qgroups - 1) // qgroups)
-    per = ((width + splits - 1) // splits + 127) // 128 * 128
-    splits = (width + per - 1) // per
-    splits = (splits + 7) // 8 * 8 if splits >= 8 else splits
-    rec = workspace[records_at:records_at + rows * splits * 8].view(torch.int32).view(rows, splits, 2)
+    layout = indexer.select_layout(layer.device, rows, tokens)
+    splits, per, at = layout.splits, layout.per, layout.records_at
+    rec = workspace[at:at + rows * splits * 8].view(torch.int32).view(rows, splits, 2)
     live = [sp for sp in range(splits) if sp * per < tokens]
     candidates = int(rec[:, live, 0].sum().item())
     spilled = int((rec[:, live, 1] != 0x7FFFFFFF).sum().item())

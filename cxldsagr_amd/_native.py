@@ -42,6 +42,7 @@ SIGNATURES = {
     "dsa_indexer_topk_fp8": [_ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _i64, _i64, _i64, _ptr,
                              _ptr, _i64, _ptr, _ptr, _i64, _ptr, _i64, _ptr],
     "dsa_indexer_select_workspace_bytes": [_i64, _i64, _i64, ctypes.POINTER(ctypes.c_int64)],
+    "dsa_indexer_select_layout": [_i64, _i64, _i64, ctypes.POINTER(ctypes.c_int64)],
     "dsa_indexer_floors_fp8": [_ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _i64, _i64, _i64, _ptr,
                                _ptr],
     "dsa_indexer_logits_fp8_emit": [_ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _i64, _i64, _i64,

@@ -849,6 +849,18 @@ extern "C" int dsa_indexer_select_workspace_bytes(int64_t rows, int64_t columns,
   return kOk;
 }
 
+extern "C" int dsa_indexer_select_layout(int64_t rows, int64_t columns, int64_t list_cap,
+                                         int64_t* layout) {
+  using namespace dsa;
+  DSA_CHECK_ARG(rows >= 0 && rows < 0x7FFFFFFF && columns >= 1 && columns < 0x7FFFFFFF - 256 &&
+                    list_cap >= 0 && layout != nullptr,
+                "invalid indexer select layout query");
+  const EmitLayout l = emit_layout(rows, columns, list_cap);
+  const int64_t parts[6] = {l.plan.splits, l.plan.per, l.cap, l.records_offset, l.lists_offset, l.bytes};
+  for (int i = 0; i < 6; ++i) layout[i] = parts[i];
+  return kOk;
+}
+
 extern "C" int dsa_indexer_floors_fp8(const void* q, const void* k, const float* weights,
                                       const float* kscale, const int32_t* starts,
                                       const int32_t* ends, int64_t query_start, int64_t rows,

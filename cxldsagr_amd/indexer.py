@@ -18,6 +18,7 @@ no host synchronisation.
 """
 
 import ctypes
+from typing import NamedTuple
 
 import torch
 
@@ -292,6 +293,27 @@ def layer_select(index_q, index_k, weights, index_keys, index_scales, position, 
             scores.data_ptr(), scratch.data_ptr(), needed, workspace.data_ptr(),
             workspace.numel(), stream)
     return ids
+
+
+class SelectLayout(NamedTuple):
+    """Parts of the ``select_topk`` workspace (``dsa_indexer_select_layout``):
+    records int32 ``[rows, splits, 2]`` at ``records_at`` ({keys listed, first
+    column stored in full or INT32_MAX}), lists of ``cap`` keys at ``lists_at``;
+    split s covers columns ``s * per`` on."""
+    splits: int
+    per: int
+    cap: int
+    records_at: int
+    lists_at: int
+    nbytes: int
+
+
+def select_layout(device, rows, columns, list_cap=0):
+    """The ``SelectLayout`` of ``select_topk`` on a device."""
+    parts = (ctypes.c_int64 * 6)()
+    with _native.on_device(device):
+        _native.call("dsa_indexer_select_layout", rows, columns, list_cap, parts)
+    return SelectLayout(*parts)
 
 
 def select_floors_buffer(device, rows, columns):

@@ -246,6 +246,11 @@ int dsa_indexer_topk_fp8(const void* q, const void* k, const float* weights, con
  */
 int dsa_indexer_select_workspace_bytes(int64_t rows, int64_t columns, int64_t list_cap,
                                        int64_t* bytes);
+/* Where the workspace's parts lie, for a reader of the records: layout =
+ * {splits (the stride of the records and lists), keys per split, keys per list,
+ * byte offset of the records, of the lists, bytes}. Split s holds columns
+ * s * per .. (s + 1) * per - 1; splits past the last column hold no records. */
+int dsa_indexer_select_layout(int64_t rows, int64_t columns, int64_t list_cap, int64_t* layout);
 int dsa_indexer_floors_fp8(const void* q, const void* k, const float* weights, const float* kscale,
                            const int32_t* starts, const int32_t* ends, int64_t query_start,
                            int64_t rows, int64_t columns, int64_t topk, uint32_t* floors,

@@ -52,17 +52,10 @@ def _same(got, want):
 
 
 def _split_plan(rows, columns, device):
-    """The logits launcher's key splits (logits.hip split_plan): (splits, per)."""
-    ldo = (columns + 255) // 256 * 256
-    cus = torch.cuda.get_device_properties(device).multi_processor_count
-    qgroups = (rows + 15) // 16
-    splits = max(1, (cus + qgroups - 1) // qgroups)
-    per = (ldo + splits - 1) // splits
-    per = (per + 127) // 128 * 128
-    splits = (ldo + per - 1) // per
-    if splits >= 8:
-        splits = (splits + 7) // 8 * 8
-    return splits, per
+    """The logits launcher's key splits: (splits, per)."""
+    from cxldsagr_amd import indexer
+
+    return indexer.select_layout(device, rows, columns)[:2]
 
 
 def _radix(values):
@@ -128,6 +121,36 @@ def test_select_config1_lists_only_candidates(gpu):
     for sp in live:
         listed = candidates[:, sp * per:min(columns, (sp + 1) * per)].sum(dim=1)
         assert torch.equal(rec[:, sp, 0].to(torch.int64), listed)
+
+
+@pytest.mark.parametrize("rows,columns", [(300, 65664), (700, 30000), (40, 20000), (1000, 40000)])
+def test_select_layout_finds_the_records(gpu, rows, columns):
+    """The records of splits that did not spill, read where the layout says,
+    count the scores at or above the floors."""
+    from cxldsagr_amd import _native, indexer
+
+    start = columns - rows
+    q, k, w, s = _inputs(rows, columns, gpu, seed=5)
+    scores = indexer.logits(q, k, w, s, start)
+    indexer.select_topk(q, k, w, s, start, 2048)
+    torch.cuda.synchronize()
+    workspace, _ = indexer._SELECT_BUFFERS[(gpu.index, _native.stream_of(gpu).value)]
+    layout = indexer.select_layout(gpu, rows, columns)
+    assert layout.nbytes == _native.size_of("dsa_indexer_select_workspace_bytes", gpu.index, rows, columns, 0)
+    pair = workspace[:8 * rows].view(torch.int32).view(rows, 2).to(torch.int64) & 0xFFFFFFFF
+    floors = pair.min(dim=1).values
+    at, splits = layout.records_at, layout.splits
+    rec = workspace[at:at + rows * splits * 8].view(torch.int32).view(rows, splits, 2)
+    hits = _radix(scores) >= floors[:, None]
+    read = 0
+    for sp in range(splits):
+        if sp * layout.per >= columns:
+            continue
+        listed = hits[:, sp * layout.per:min(columns, (sp + 1) * layout.per)].sum(dim=1)
+        whole = (floors != 0) & (rec[:, sp, 1] == 0x7FFFFFFF)
+        assert torch.equal(rec[whole, sp, 0].to(torch.int64), listed[whole])
+        read += int(whole.sum())
+    assert read > rows  # most splits list what they hold
 
 
 def test_select_forced_recompute(gpu):
