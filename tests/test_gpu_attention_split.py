@@ -90,8 +90,7 @@ def test_negative_and_zero_scales_take_one_launch(gpu):
 def test_rows_that_end_in_padding_equal_their_short_selections(gpu, heads):
     """Rows stop at their last id in range: a full round of rows whose ids end
     at every edge of the 64-key step has, row by row, the bits of the same ids
-    without the padding (a page table shorter than the ids' range and ids past
-    the cache count as padding)."""
+    without the padding (-1, or ids past the records)."""
     from cxldsagr_amd.attention import sparse_mla
 
     gen = torch.Generator(device=gpu).manual_seed(11)
@@ -108,6 +107,50 @@ def test_rows_that_end_in_padding_equal_their_short_selections(gpu, heads):
         want = (sparse_mla(q[r:r + 1], kv, ids[r:r + 1, :end].contiguous(), SCALE)[0] if end
                 else torch.zeros_like(got[r]))
         assert torch.equal(got[r].view(torch.int16), want.view(torch.int16)), end
+
+
+@pytest.mark.parametrize("heads", [64, 192])
+def test_paged_rows_that_end_in_padding(gpu, heads):
+    """The same over the fp8 paged cache, whose rows stop by a look-ahead of
+    their own: -1, ids past n_tokens (the page table covers more) and ids on
+    pages outside the cache, which do not stop a row. The oracle of the
+    dequantised records has the same rows (tolerance: a bf16 output and P)."""
+    import numpy as np
+
+    from cxldsagr_amd.attention import pack_kv_fp8, sparse_mla_fp8_paged
+    from oracle import kv_fp8 as okv
+    from oracle import sparse_mla as omla
+
+    gen = torch.Generator(device=gpu).manual_seed(12)
+    rows, selected, tokens, pages = 256 if heads == 64 else 85, 300, 1000, 16
+    kv = torch.randn(tokens, 576, generator=gen, device=gpu).bfloat16()
+    table = torch.randperm(pages, generator=gen, device=gpu).int()
+    cache = torch.zeros(pages, 64, 656, dtype=torch.uint8, device=gpu)
+    pack_kv_fp8(kv, cache, table)
+    records = okv.logical_records(cache.cpu().numpy(), table.cpu().numpy(), tokens)
+    table = torch.cat((table, torch.zeros(4, dtype=torch.int32, device=gpu)))
+    table[3], table[7] = pages, -1  # outside the cache
+    outside = torch.zeros(tokens, dtype=torch.bool, device=gpu)
+    outside[192:256] = outside[448:512] = True
+    q = torch.randn(rows, heads, 576, generator=gen, device=gpu).bfloat16()
+    ids = torch.randint(0, tokens, (rows, selected), generator=gen, device=gpu).int()
+    ids[:, 5::11] = 200  # on a page outside
+    ends = [0, 1, 31, 32, 33, 63, 64, 65, 127, 128, 129, 191, 192, 255, 256, 257, 299, 300]
+    fills = [-1, tokens, 470]
+    for r in range(rows):
+        ids[r, ends[r % len(ends)]:] = fills[r % 3]
+    got = sparse_mla_fp8_paged(q, cache, table, ids, SCALE, n_tokens=tokens)
+    for r in range(54):  # every end with every filling
+        end = ends[r % len(ends)]
+        want = (sparse_mla_fp8_paged(q[r:r + 1], cache, table, ids[r:r + 1, :end].contiguous(),
+                                     SCALE, n_tokens=tokens)[0] if end else torch.zeros_like(got[r]))
+        assert torch.equal(got[r].view(torch.int16), want.view(torch.int16)), (r, end)
+    valid = (ids >= 0) & (ids < tokens)
+    valid &= ~outside[ids.clamp(0, tokens - 1).long()]
+    sample = list(range(0, 54, 5))
+    _, ref = omla.sparse_mla(q[sample].float().cpu().numpy(), records,
+                             torch.where(valid, ids, -1)[sample].cpu().numpy(), SCALE)
+    np.testing.assert_allclose(got[sample].float().cpu().numpy(), ref, atol=4e-3, rtol=2e-2)
 
 
 @pytest.mark.parametrize("fewer,more,heads,selected", [(12, 16, 128, 2048), (26, 32, 128, 2048),
