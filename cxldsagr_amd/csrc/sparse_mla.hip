@@ -333,8 +333,8 @@ __global__ __launch_bounds__(kThreads, 1) void sparse_mla_fwd(
   // ahead; the four lanes of a key store the same value), and stages block 0;
   // the score waves load their Q beside that. With the ring filled by all
   // waves and Q loaded behind its barrier, 16.7k of a 2,048-key tile's 185k
-  // cycles passed before the first step, now 11.7k (1,024 rows of 128 heads:
-  // 683 -> 621 us).
+  // cycles passed before the first step, then 11.7k (1,024 rows of 128 heads,
+  // eight rounds: 648 -> 636 us, with 64 keys 109.7 -> 106.0).
   if (!scorer) {
     int32_t rows0[kRingAhead], pages0[kRingAhead];
 #pragma unroll
@@ -716,8 +716,8 @@ __global__ __launch_bounds__(kThreads, 1) void sparse_mla_fwd(
     // Two dim tiles at a time: the row groups swap halves, so that a lane
     // holds 8 consecutive dims (of tile m + (g & 1)) and a head's 64 bytes go
     // out in one instruction. With 8 bytes a lane (32 of a head) the stores
-    // took 7.5k cycles to land, now 3.9k (1,024 rows of 128 heads and 2,048
-    // keys: 621 -> 610 us, 64 keys: 104 -> 92 us).
+    // took 7.5k cycles to land, now 3.9k (1,024 rows of 128 heads: 636 -> 631
+    // us, with 64 keys 106.0 -> 94.4).
     uint16_t* obase = out + ((row * heads + head0 + c) * kVDim) + dim0 + 16 * (g & 1) + 8 * (g >> 1);
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
@@ -752,23 +752,24 @@ __global__ __launch_bounds__(kThreads, 1) void sparse_mla_fwd(
 //   writes the blocks' scores (fp32, -inf at padding) in the order of the PV
 //   operands, and each block's maximum per head.
 // * mla_values: the value dims are independent of each other. A work-group
-//   takes a row, 64 heads and 64 of the 512 dims, replays the running-max
+//   takes a row, 64 heads and 64 or 128 of the 512 dims, replays the running-max
 //   chain from the block maxima, forms P^T straight in the operand registers
 //   and runs the PV products block by block, in sparse_mla_fwd's order.
 // A block without a valid key changes no sum and is skipped.
 //
-// What bounds them at few rows: mla_scores (9 us for one row of 128 heads, 16
-// for 16) is a chain of load latencies, ids -> pages -> records -> LDS, in
-// front of one to four 1,152-cycle MFMA steps; from 64 rows on (34 us) the
-// 1 MB of fp32 scores per row it writes. mla_values (24 us for one row) is
-// one wave per SIMD issuing ~65 instructions per block (~650 cycles with the
-// LDS waits).
+// What bounds them: mla_scores (9.6 us for one row of 128 heads, 16.4 for 16) is
+// a chain of load latencies, ids -> pages -> records -> LDS, in front of one to
+// eight 1,152-cycle MFMA steps. mla_values (23.0 us for one row, 25.3 for 16, 32.2 for 32
+// with 128 dims) is one wave per SIMD issuing ~65 instructions per block (~650
+// cycles with the LDS waits). The workspace holds 1 MB of fp32 scores per row of
+// 128 heads and 2,048 selected (34 MB with the maxima at the 32 rows of a quarter round).
 constexpr int kScoreThreads = 512;
 constexpr int kScoreKeys = 1024;                      // most keys per work-group of mla_scores
 constexpr int kSplitSelected = 2048;                  // widest selection of the split form
 constexpr int kValueThreads = 256;
 constexpr int kValueBlocks = 2;                       // key blocks per step of mla_values
 constexpr int kValueKeys = kValueBlocks * kBlock;
+constexpr int kValueDepth = 4;                        // steps of mla_values' loads in flight
 
 // The records of positions first + tid + kThreadsN u (u < kBatch) of a
 // selection; the zero record for padding, an id outside [0, n_tokens) or a
@@ -821,7 +822,6 @@ __global__ __launch_bounds__(kScoreThreads, 1) void mla_scores(
     const int32_t* __restrict__ indices, int64_t heads, int64_t topk, float scale_log2,
     int32_t chunks, int32_t chunk_steps, float* __restrict__ scores,
     float* __restrict__ block_max) {
-  using F = Format<kFp8>;
   constexpr int kStepBlocks = 4 / kTiles;
   constexpr int kStepKeys = kStepBlocks * kBlock;
   // Staging: kLanes lanes per key, each 16-byte pieces of its record.
@@ -1003,9 +1003,9 @@ __global__ __launch_bounds__(kScoreThreads, 1) void mla_scores(
 // One work-group: a row, 64 heads (wave w: heads 16 w .. + 15) and kDv of the
 // value dims, in steps of kValueBlocks key blocks. Latency rules it (records,
 // scores and maxima come from the last-level cache or HBM), so all loads of a
-// step go out kDepth steps ahead.
-template <bool kFp8, int kDv, int kDepth>
-__global__ __launch_bounds__(kValueThreads, kDv < 256 ? 2 : 1) void mla_values(
+// step go out kValueDepth steps ahead.
+template <bool kFp8, int kDv>
+__global__ __launch_bounds__(kValueThreads, 2) void mla_values(
     const uint8_t* __restrict__ kv, const int32_t* __restrict__ page_table, int64_t n_tokens,
     int64_t pages, const int32_t* __restrict__ indices, int64_t rows, int64_t heads, int64_t topk,
     float scale_log2, const float* __restrict__ scores, const float* __restrict__ block_max,
@@ -1016,7 +1016,7 @@ __global__ __launch_bounds__(kValueThreads, kDv < 256 ? 2 : 1) void mla_values(
   constexpr int kStride = 2 * kDv + 16;
   static_assert(kStride / 4 % 64 == 4 || kStride / 4 % 64 == 36, "bank windows of the transpose reads");
   __shared__ __align__(16) uint8_t v_lds[2][kValueKeys * kStride];
-  __shared__ uint64_t records[kSplitSelected + (kDepth + 1) * kValueKeys];  // + the look-ahead
+  __shared__ uint64_t records[kSplitSelected + (kValueDepth + 1) * kValueKeys];  // + the look-ahead
   __shared__ int32_t wave_last[kValueThreads / 64];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1037,8 +1037,8 @@ __global__ __launch_bounds__(kValueThreads, kDv < 256 ? 2 : 1) void mla_values(
   const int n_blocks = padded_blocks(topk);
 
   // Scores and maxima of this wave's 16 heads (uniform base, lane offset).
-  v4f s_lo[kDepth][kValueBlocks], s_hi[kDepth][kValueBlocks];
-  float mb[kDepth][kValueBlocks];
+  v4f s_lo[kValueDepth][kValueBlocks], s_hi[kValueDepth][kValueBlocks];
+  float mb[kValueDepth][kValueBlocks];
   // (A row's scores are n_blocks x heads x 128 bytes: 32-bit offsets.)
   const int64_t tiles16 = heads / 16;
   const uint8_t* s_base = reinterpret_cast<const uint8_t*>(scores + (row * n_blocks * tiles16 + head0 / 16) * kScoreTile);
@@ -1057,7 +1057,7 @@ __global__ __launch_bounds__(kValueThreads, kDv < 256 ? 2 : 1) void mla_values(
     int32_t last = -1;
     constexpr int kBatch = 8;
     const int total = n_blocks * kBlock;
-    for (int i = threadIdx.x; i < (kDepth + 1) * kValueKeys; i += kValueThreads)
+    for (int i = threadIdx.x; i < (kValueDepth + 1) * kValueKeys; i += kValueThreads)
       records[total + i] = (uint64_t)(uintptr_t)zero_record;
     for (int i0 = 0; i0 < total; i0 += kBatch * kValueThreads) {
       uint64_t rec[kBatch];
@@ -1077,9 +1077,9 @@ __global__ __launch_bounds__(kValueThreads, kDv < 256 ? 2 : 1) void mla_values(
   __syncthreads();
   const int last = __builtin_amdgcn_readfirstlane(
       max(max(wave_last[0], wave_last[1]), max(wave_last[2], wave_last[3])));
-  static_assert(kValueRound % (kDepth * kValueBlocks) == 0, "whole rounds of the register sets");
+  static_assert(kValueRound % (kValueDepth * kValueBlocks) == 0, "whole rounds of the register sets");
   // Steps up to the last valid position, in whole rounds of the register sets.
-  const int steps = (last + kDepth * kValueKeys) / (kDepth * kValueKeys) * kDepth;
+  const int steps = (last + kValueDepth * kValueKeys) / (kValueDepth * kValueKeys) * kValueDepth;
 
   // Staging: four lanes per key.
   static_assert(4 * kValueKeys == kValueThreads, "a step's keys by four lanes each");
@@ -1087,8 +1087,8 @@ __global__ __launch_bounds__(kValueThreads, kDv < 256 ? 2 : 1) void mla_values(
   const int j = threadIdx.x & 3;
   constexpr int kRaw = kDv / 64 * (kFp8 ? 1 : 2);
   constexpr int kScales = kFp8 ? (kDv + 127) / 128 : 1;
-  v4u raw[kDepth][kRaw];
-  float tile_scale[kDepth][kScales] = {};
+  v4u raw[kValueDepth][kRaw];
+  float tile_scale[kValueDepth][kScales] = {};
   uint64_t rec_next = records[kk];  // of the next step to fetch
   const int scale_at = kVDim + 4 * (d0 / 128) - d0;  // from the record's first value byte here
   auto fetch = [&](int t, int set) __attribute__((always_inline)) {
@@ -1132,7 +1132,7 @@ __global__ __launch_bounds__(kValueThreads, kDv < 256 ? 2 : 1) void mla_values(
   float alpha = 1.0f;
   auto softmax = [&](float mx, const v4f& lo, const v4f& hi) __attribute__((always_inline)) -> v8bf {
     const bool need = (mx > m_run + kRescaleThreshold) | ((m_run == neg_inf) & (mx != neg_inf));
-    const float m_new = need & (mx > m_run) ? mx : m_run;
+    const float m_new = (need & (mx > m_run)) ? mx : m_run;
     alpha = need ? __builtin_amdgcn_exp2f(m_run - m_new) : 1.0f;
     m_run = m_new;
     const float neg_m = m_run == neg_inf ? 0.0f : -m_run;
@@ -1142,7 +1142,7 @@ __global__ __launch_bounds__(kValueThreads, kDv < 256 ? 2 : 1) void mla_values(
   };
   if (steps > 0) {
 #pragma unroll
-    for (int u = 0; u < kDepth; ++u) {
+    for (int u = 0; u < kValueDepth; ++u) {
       fetch(u, u);
 #pragma unroll
       for (int b = 0; b < kValueBlocks; ++b) load_scores(u, b, u);
@@ -1150,13 +1150,13 @@ __global__ __launch_bounds__(kValueThreads, kDv < 256 ? 2 : 1) void mla_values(
     // The softmax runs one block ahead of the PV products: its VALU work
     // fills the LDS latency and the MFMAs of the block before.
     v8bf p_next = softmax(mb[0][0], s_lo[0][0], s_hi[0][0]);
-    for (int t0 = 0; t0 < steps; t0 += kDepth) {
+    for (int t0 = 0; t0 < steps; t0 += kValueDepth) {
 #pragma unroll
-      for (int u = 0; u < kDepth; ++u) {
+      for (int u = 0; u < kValueDepth; ++u) {
         const int t = t0 + u;
         stage(t, u);  // the buffer's last readers passed the previous barrier
         __builtin_amdgcn_sched_barrier(0);
-        fetch(t + kDepth, u);
+        fetch(t + kValueDepth, u);
         lds_barrier();
         const uint32_t vb = v_lane + (uint32_t)(t & 1) * (uint32_t)sizeof(v_lds[0]);
 #pragma unroll
@@ -1175,7 +1175,7 @@ __global__ __launch_bounds__(kValueThreads, kDv < 256 ? 2 : 1) void mla_values(
             v1[m] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s)(uintptr_t)(at + 16 * kStride));
           }
           // The next block's scores: in this step's set or the next one's.
-          const int nu = b + 1 < kValueBlocks ? u : (u + 1) % kDepth;
+          const int nu = b + 1 < kValueBlocks ? u : (u + 1) % kValueDepth;
           const int nb = b + 1 < kValueBlocks ? b + 1 : 0;
           v4u p_regs = __builtin_bit_cast(v4u, softmax(mb[nu][nb], s_lo[nu][nb], s_hi[nu][nb]));
           asm volatile("" : "+v"(p_regs));  // here, ahead of the MFMAs that wait for the V^T reads
@@ -1191,7 +1191,7 @@ __global__ __launch_bounds__(kValueThreads, kDv < 256 ? 2 : 1) void mla_values(
         // here, and the copies would wait for them.
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int b = 0; b < kValueBlocks; ++b) load_scores(t + kDepth, b, u);
+        for (int b = 0; b < kValueBlocks; ++b) load_scores(t + kValueDepth, b, u);
       }
     }
   }
@@ -1280,7 +1280,7 @@ int launch_split(const MlaPlan& p, const uint16_t* q, int64_t heads, const uint8
                      (int32_t)chunks, (int32_t)chunk, scores, block_max);
   DSA_CHECK_LAUNCH("sparse MLA scores");
   const int64_t groups = (rows * (heads / 64) + 7) / 8;
-  hipLaunchKernelGGL((p.dv == 64 ? mla_values<kFp8, 64, 4> : mla_values<kFp8, 128, 4>),
+  hipLaunchKernelGGL((p.dv == 64 ? mla_values<kFp8, 64> : mla_values<kFp8, 128>),
                      dim3((unsigned)(groups * 8 * (kVDim / p.dv))), dim3(kValueThreads), 0, stream,
                      kv, page_table, n_tokens, pages, indices, rows, heads, topk, scale_log2,
                      scores, block_max, out);
