@@ -236,7 +236,9 @@ class DSALayer:
     def _prologue(self, index_q, index_k, weights, kv, position, floors=None):
         """Q quantisation + weight fold, new index K into the cache and the new
         KV records into the fp8 paged cache, in one launch (``index_prologue``).
-        Returns ``(q8, folded, q_fold)``."""
+        Returns ``(q8, folded, q_fold)``. The stage by itself, for timing it and
+        comparing its outputs: ``forward`` queues the same launch together with
+        the logits and the top-k (``indexer.layer_select``)."""
         return index_prologue(index_q, index_k, weights, self.index_keys, self.index_scales,
                               position, self.topk, floors, kv=kv, page_table=self.page_table,
                               kv_cache=self.kv_cache)
