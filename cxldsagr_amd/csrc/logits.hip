@@ -770,6 +770,41 @@ int check_emit_buffers(int64_t rows, int64_t columns, int64_t list_cap, const fl
   return kOk;
 }
 
+// The launches of the candidate calls, on checked arguments and the layout of
+// check_emit_buffers (choosing the key splits is host time: once per call).
+int launch_emit_logits(const void* q, const void* k, const float* weights, const float* kscale,
+                       const int32_t* starts, const int32_t* ends, int64_t query_start,
+                       int64_t rows, int64_t columns, const float* q_fold, float* scores,
+                       const EmitLayout& l, void* workspace, hipStream_t stream) {
+  uint8_t* base = static_cast<uint8_t*>(workspace);
+  EmitArgs emit{reinterpret_cast<const uint32_t*>(base),
+                reinterpret_cast<uint64_t*>(base + l.lists_offset),
+                reinterpret_cast<uint32_t*>(base + l.records_offset), (int32_t)l.cap,
+                (int32_t)l.plan.splits};
+  hipLaunchKernelGGL(logits_fp8_mfma<kModeEmit>, dim3(l.plan.grid()),
+                     dim3(kThreads), 0, stream, static_cast<const uint8_t*>(q),
+                     static_cast<const uint8_t*>(k), weights, kscale, starts, ends, query_start,
+                     rows, columns, (columns + 255) / 256 * 256, l.plan.per, q_fold, scores, nullptr,
+                     emit, (uint32_t)l.plan.qgroups, (uint32_t)l.plan.live);
+  DSA_CHECK_LAUNCH("indexer logits (candidates)");
+  return kOk;
+}
+
+int launch_emit_topk(const void* q, const void* k, const float* weights, const float* kscale,
+                     const int32_t* starts, const int32_t* ends, int64_t query_start, int64_t rows,
+                     int64_t columns, const float* q_fold, float* scores, int64_t topk,
+                     float* values, int32_t* indices, int64_t out_ld, const EmitLayout& l,
+                     const void* workspace, hipStream_t stream) {
+  const uint8_t* base = static_cast<const uint8_t*>(workspace);
+  return topk_from_candidates(
+      static_cast<const uint8_t*>(q), static_cast<const uint8_t*>(k), weights, kscale, starts,
+      ends, query_start, q_fold, scores, rows, columns, (columns + 255) / 256 * 256, topk, values,
+      indices, out_ld, reinterpret_cast<const uint32_t*>(base),
+      reinterpret_cast<const uint32_t*>(base + l.records_offset),
+      reinterpret_cast<const uint64_t*>(base + l.lists_offset), l.plan.splits, l.plan.per, l.cap,
+      stream);
+}
+
 }  // namespace
 }  // namespace dsa
 
@@ -895,18 +930,8 @@ extern "C" int dsa_indexer_logits_fp8_emit(const void* q, const void* k, const f
   EmitLayout l;
   status = check_emit_buffers(rows, columns, list_cap, scores, workspace, workspace_bytes, &l);
   if (status != kOk) return status;
-  uint8_t* base = static_cast<uint8_t*>(workspace);
-  EmitArgs emit{reinterpret_cast<const uint32_t*>(base),
-                reinterpret_cast<uint64_t*>(base + l.lists_offset),
-                reinterpret_cast<uint32_t*>(base + l.records_offset), (int32_t)l.cap,
-                (int32_t)l.plan.splits};
-  hipLaunchKernelGGL(logits_fp8_mfma<kModeEmit>, dim3(l.plan.grid()),
-                     dim3(kThreads), 0, stream, static_cast<const uint8_t*>(q),
-                     static_cast<const uint8_t*>(k), weights, kscale, starts, ends, query_start,
-                     rows, columns, ldo, l.plan.per, q_fold, scores, nullptr, emit,
-                     (uint32_t)l.plan.qgroups, (uint32_t)l.plan.live);
-  DSA_CHECK_LAUNCH("indexer logits (candidates)");
-  return kOk;
+  return launch_emit_logits(q, k, weights, kscale, starts, ends, query_start, rows, columns, q_fold,
+                            scores, l, workspace, stream);
 }
 
 extern "C" int dsa_indexer_emit_topk(const void* q, const void* k, const float* weights,
@@ -926,14 +951,8 @@ extern "C" int dsa_indexer_emit_topk(const void* q, const void* k, const float* 
   EmitLayout l;
   status = check_emit_buffers(rows, columns, list_cap, scores, workspace, workspace_bytes, &l);
   if (status != kOk) return status;
-  const uint8_t* base = static_cast<const uint8_t*>(workspace);
-  return topk_from_candidates(
-      static_cast<const uint8_t*>(q), static_cast<const uint8_t*>(k), weights, kscale, starts,
-      ends, query_start, q_fold, scores, rows, columns, (columns + 255) / 256 * 256, topk, values,
-      indices, out_ld, reinterpret_cast<const uint32_t*>(base),
-      reinterpret_cast<const uint32_t*>(base + l.records_offset),
-      reinterpret_cast<const uint64_t*>(base + l.lists_offset), l.plan.splits, l.plan.per, l.cap,
-      stream);
+  return launch_emit_topk(q, k, weights, kscale, starts, ends, query_start, rows, columns, q_fold,
+                          scores, topk, values, indices, out_ld, l, workspace, stream);
 }
 
 // Floors, candidate logits and the top-k from the candidates, in one call.
@@ -958,13 +977,11 @@ extern "C" int dsa_indexer_select_fp8(const void* q, const void* k, const float*
   status = dsa_indexer_floors_fp8(q, k, weights, kscale, starts, ends, query_start, rows, columns,
                                   topk, static_cast<uint32_t*>(workspace), stream);
   if (status != kOk) return status;
-  status = dsa_indexer_logits_fp8_emit(q, k, weights, kscale, starts, ends, query_start, rows,
-                                       columns, ldo, q_fold, scores, 0, workspace, workspace_bytes,
-                                       stream);
+  status = launch_emit_logits(q, k, weights, kscale, starts, ends, query_start, rows, columns,
+                              q_fold, scores, l, workspace, stream);
   if (status != kOk) return status;
-  return dsa_indexer_emit_topk(q, k, weights, kscale, starts, ends, query_start, rows, columns,
-                               q_fold, scores, topk, values, indices, out_ld, 0, workspace,
-                               workspace_bytes, stream);
+  return launch_emit_topk(q, k, weights, kscale, starts, ends, query_start, rows, columns, q_fold,
+                          scores, topk, values, indices, out_ld, l, workspace, stream);
 }
 
 // A layer step's indexer half in one call: the prologue launch with floors,
@@ -1034,12 +1051,10 @@ extern "C" int dsa_layer_indexer_fp8(const void* q, int64_t rows, const float* w
       kv ? rows : 0, kv ? position : 0, page_table, kv ? pages : 0, cache, nullptr, index_keys,
       index_scales, position, topk, static_cast<uint32_t*>(workspace), stream);
   if (status != kOk) return status;
-  status = dsa_indexer_logits_fp8_emit(base, index_keys, folded, index_scales, nullptr, nullptr,
-                                       position, rows, columns, ldo, q_fold, scores, 0, workspace,
-                                       workspace_bytes, stream);
+  status = launch_emit_logits(base, index_keys, folded, index_scales, nullptr, nullptr, position,
+                              rows, columns, q_fold, scores, l, workspace, stream);
   if (status != kOk) return status;
-  return dsa_indexer_emit_topk(base, index_keys, folded, index_scales, nullptr, nullptr, position,
-                               rows, columns, q_fold, scores, topk,
-                               reinterpret_cast<float*>(base + at.values), indices, count, 0,
-                               workspace, workspace_bytes, stream);
+  return launch_emit_topk(base, index_keys, folded, index_scales, nullptr, nullptr, position, rows,
+                          columns, q_fold, scores, topk, reinterpret_cast<float*>(base + at.values),
+                          indices, count, l, workspace, stream);
 }

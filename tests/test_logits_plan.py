@@ -78,3 +78,21 @@ def test_pairs_are_dealt_once_and_evenly(plan_library, rows, ldo):
     seen = np.clip(ends[None, :] - per * np.arange(live)[:, None], 0, per)
     work = (on * seen).sum((1, 2))
     assert work.max() <= 1.1 * work.mean() + per * (qgroups if live >= 8 else 1), work
+
+
+@pytest.mark.parametrize("cus", [256, 304, 7])
+def test_the_plan_is_the_cheapest_of_all_split_counts(plan_library, cus):
+    """Each split length is looked at once; the result is that of every count in
+    turn, the first of those that cost the same."""
+    rng = np.random.default_rng(cus)
+    ldos = np.concatenate([256 * np.arange(1, 40), 256 * rng.integers(40, 4200, 60)])
+    out = (ctypes.c_int64 * 5)()
+    for ldo in ldos.tolist():
+        rows = int(rng.choice([1, 16, 17, 100, 128, 700, 2048, 9000]))
+        stages, qgroups = (ldo + 127) // 128, (rows + 15) // 16
+        s = np.arange(1, min(stages, cus) + 1)
+        per = -(-stages // s)
+        rounds = -(-(-(-stages // per) * qgroups) // cus)
+        best = per[np.argmin(rounds * (8.0 + 3.0 * per))] * 128
+        plan_library.plan(ctypes.c_int64(rows), ctypes.c_int64(ldo), ctypes.c_int64(cus), out)
+        assert out[2] == best, (rows, ldo)
