@@ -134,23 +134,24 @@ def indexer_stage_calls(layer, tokens, topk, q8, folded, q_fold, workspace):
     return logits_fn, topk_fn, ids
 
 
-# "marker" is an empty bracket: two events recorded back to back, the cost
-# one event marker adds to each stage interval.
-STAGES = ("marker", "prologue", "logits", "topk", "sparse_mla")
+STAGES = ("prologue", "logits", "topk", "sparse_mla")
+LEAD_STEPS = 20  # untimed: the first steps after a synchronisation wait for the host
 
 
-def in_layer_stage_us(torch, layer, history, tokens, topk, iters, args):
+def in_layer_stage_us(torch, step, layer, history, tokens, topk, iters, args):
     """Average duration of each stage of the layer step, from HIP events recorded
     between its launches on the current stream (the same launches, in the same
     order, as DSALayer.forward, which queues the indexer's three in one native
-    call; the per-row floors are part of the prologue launch), after an empty
-    bracket that measures what one event marker adds to a stage. Also returns the candidate keys the indexer step listed and
-    the key splits that spilled."""
+    call; the per-row floors are part of the prologue launch). "marker" is what
+    the events add to a stage: a quarter of what these steps take above the plain
+    ``step``, timed just ahead of them on the same full queue. Also returns the
+    candidate keys the indexer step listed and the key splits that spilled."""
     index_q, index_k, weights, mla_q, kv = args
     fused = layer._fused_prologue_applies(index_q, index_k, weights, kv)
     stream = torch.cuda.current_stream()
     marks = [[torch.cuda.Event(enable_timing=True) for _ in range(len(STAGES) + 1)]
-             for _ in range(iters)]
+             for _ in range(LEAD_STEPS + iters)]
+    plain = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
     rows = len(index_q)
     workspace = select_workspace(rows, tokens, layer.device)
     floors = workspace[:8 * rows].view(torch.int32).view(rows, 2)
@@ -172,18 +173,22 @@ def in_layer_stage_us(torch, layer, history, tokens, topk, iters, args):
     logits_fn, topk_fn, ids = indexer_stage_calls(
         layer, tokens, topk, q8, folded, q_fold, workspace)
     torch.cuda.synchronize()
+    for i in range(LEAD_STEPS + iters):
+        if i == LEAD_STEPS:
+            plain[0].record(stream)
+        step()
+    plain[1].record(stream)
     for ev in marks:
         layer.written = history
         ev[0].record(stream)
-        ev[1].record(stream)
         prologue()
-        ev[2].record(stream)
+        ev[1].record(stream)
         logits_fn()
-        ev[3].record(stream)
+        ev[2].record(stream)
         topk_fn()
-        ev[4].record(stream)
+        ev[3].record(stream)
         layer._attend(mla_q, ids, tokens)
-        ev[5].record(stream)
+        ev[4].record(stream)
     torch.cuda.synchronize()
     # Candidates listed per row (records [rows][splits][2] after the floors).
     layout = indexer.select_layout(layer.device, rows, tokens)
@@ -192,8 +197,10 @@ def in_layer_stage_us(torch, layer, history, tokens, topk, iters, args):
     live = [sp for sp in range(splits) if sp * per < tokens]
     candidates = int(rec[:, live, 0].sum().item())
     spilled = int((rec[:, live, 1] != 0x7FFFFFFF).sum().item())
-    times = {name: sum(ev[i].elapsed_time(ev[i + 1]) for ev in marks) * 1e3 / iters
+    times = {name: sum(ev[i].elapsed_time(ev[i + 1]) for ev in marks[LEAD_STEPS:]) * 1e3 / iters
              for i, name in enumerate(STAGES)}
+    step_us = plain[0].elapsed_time(plain[1]) * 1e3 / iters
+    times["marker"] = max(0.0, (sum(times.values()) - step_us) / len(STAGES))
     return times, candidates, spilled
 
 
@@ -359,11 +366,12 @@ def main():
     step()  # leave the layer as the plain step left it
     torch.cuda.synchronize()
     in_layer, candidates, spilled = in_layer_stage_us(
-        torch, layer, history, tokens, topk, args.steps,
+        torch, step, layer, history, tokens, topk, args.steps,
         (index_q, index_k_new, weights, mla_q, kv_new))
     # Kernel figures are the launches inside the layer step (the clock of the
     # timed region), each stage's event interval less the cost of one marker
-    # (the empty bracket); the isolated stage loops are reported beside them.
+    # (its share of what the events add to a step); the isolated stage loops are
+    # reported beside them.
     kernel_us = dict(isolated_us)
     kernel_us.update({name: us - in_layer["marker"] for name, us in in_layer.items()})
     kernel_us["marker"] = in_layer["marker"]
@@ -400,7 +408,7 @@ def main():
         # floors.
         "prologue": {"us": round(kernel_us["prologue"], 2), "with_floors": True},
         # Each stage's event interval before the marker is taken off.
-        "stage_us": {name: round(in_layer[name], 2) for name in STAGES[1:]},
+        "stage_us": {name: round(in_layer[name], 2) for name in STAGES},
         # Algorithmic bytes of the producer launch: per 128-value row 256 B in,
         # 128 B codes + 4 B scale out, 256 B of its RoPE row; per Q row 4 B head
         # logit in + 4 B weight out; the partial folded queries; per KV token
@@ -412,14 +420,13 @@ def main():
         },
         "isolated_us": {name: round(us, 2) for name, us in isolated_us.items()},
         # The stage intervals come from HIP events recorded between the
-        # layer's launches, so each carries one marker (`marker_us`, an empty
-        # bracket timed the same way): they sum above `value`, the plain
-        # step; the kernel figures above have the marker taken off, and sum
-        # below `value` by the launch gaps of the plain step.
+        # layer's launches, so each carries one marker (`marker_us`): they sum
+        # above `value`, the plain step; the kernel figures above have the
+        # marker taken off and sum to the plain step, launch gaps included.
         "marker_us": round(kernel_us["marker"], 2),
-        "stage_sum_us": round(sum(in_layer[name] for name in STAGES[1:]), 2),
-        "kernel_sum_us": round(sum(kernel_us[name] for name in STAGES[1:]), 2),
-        "stage_note": "kernel us = in-layer stage interval less one event marker",
+        "stage_sum_us": round(sum(in_layer[name] for name in STAGES), 2),
+        "kernel_sum_us": round(sum(kernel_us[name] for name in STAGES), 2),
+        "stage_note": "kernel us = in-layer stage interval less its share of what the events add to a step",
     }
     dominant = max(("logits", "topk", "sparse_mla"), key=lambda k: kernel_us[k])
     traffic = None
@@ -556,15 +563,15 @@ def config4_layer(torch, args, formats=("fp8_paged", "bf16")):
             step()
         layer_us = event_time_us(torch, step, args.steps)
         times, candidates, spilled = in_layer_stage_us(
-            torch, layer, history, tokens, topk, args.steps,
+            torch, step, layer, history, tokens, topk, args.steps,
             (index_q, index_k_new, weights, mla_q, kv_new))
         pairs = queries * history + queries * (queries + 1) // 2
         logits_flop = 2 * 64 * 128 * pairs
         mla_flop = 2 * queries * topk * 128 * (576 + 512)
         record = 656 if kv_format == "fp8_paged" else 1152
         ids = selection.token_ids
-        # Kernel estimates: each stage interval less one event marker.
-        kernel = {name: times[name] - times["marker"] for name in STAGES[1:]}
+        # Kernel estimates: each stage interval less its share of what the events add.
+        kernel = {name: times[name] - times["marker"] for name in STAGES}
         if reference is None:
             reference = mla_reference_f32(torch, mla_q, kv_all, ids, sample_rows, layer.scale)
         outputs[kv_format] = (out[sample_rows].float(), ids)
@@ -572,7 +579,7 @@ def config4_layer(torch, args, formats=("fp8_paged", "bf16")):
             "layer_us": round(layer_us, 2),
             "kernel_us": {name: round(us, 2) for name, us in kernel.items()},
             "stage_us": {name: round(us, 2) for name, us in times.items()},
-            "stage_note": "kernel us = in-layer stage interval less one event marker (stage 'marker')",
+            "stage_note": "kernel us = in-layer stage interval less its share of what the events add to a step ('marker')",
             "candidates": candidates,
             "spilled_splits": spilled,
             "logits_frac_fp8_peak": round(logits_flop / kernel["logits"] / 1e6 / PEAKS["fp8_TFLOPs"], 4),
