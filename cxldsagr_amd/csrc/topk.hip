@@ -872,7 +872,7 @@ constexpr int kListCap = kMaxK + kRefineCap;  // candidates a row may list
 constexpr int kWaveCap = 1024;                // candidates a wave stages in LDS
 constexpr uint32_t kOverflow = 0x40000000u;   // added to a row's fill by an overflowing part
 constexpr int kSortCap = kListCap;  // candidates the one-pass counting sort takes
-constexpr int kSortBins = 4096;     // its linear buckets
+constexpr int kSortBins = 4096;     // its buckets
 constexpr uint32_t kSortBucketMax = 128;  // keys per bucket it ranks by comparison
 constexpr int kSortPerThread = kSortCap / kThreads;
 // List slots per thread the candidate top-k loads before it knows the lists'

@@ -233,7 +233,7 @@ int dsa_indexer_topk_fp8(const void* q, const void* k, const float* weights, con
  * `scores` is f32 [rows, ldo] with ldo = columns rounded up to 256: scratch
  * that holds only stored rows and spilled columns afterwards. q_fold as for
  * dsa_indexer_logits_fp8_folded (may be NULL). list_cap = 0 picks the list
- * length per (row, split) (an eighth of the split); a smaller one makes
+ * length per (row, split) (an eighth of the split, at least 256 or all of it); a smaller one makes
  * splits spill earlier (for tests). The workspace (256-byte aligned, size
  * from dsa_indexer_select_workspace_bytes with the same rows, columns and
  * list_cap on the same device) holds floors u32 [rows][2] (a row's floor is
