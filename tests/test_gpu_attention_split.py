@@ -157,8 +157,7 @@ def test_paged_rows_that_end_in_padding(gpu, heads):
                                                        (24, 32, 128, 1024), (24, 32, 64, 2048)])
 def test_fewer_rows_take_no_longer(gpu, fewer, more, heads, selected):
     """The score launch's runs fit one round of work-groups for every row count
-    (fewer rows had taken 1.10 to 1.13 times as long as more, and take 0.92 to 1.0;
-    the bound lies between, as far from both as the host's noise allows)."""
+    (fewer rows had taken 1.10 to 1.13 times as long as more, and take 0.90 to 0.92)."""
     from cxldsagr_amd.attention import sparse_mla
 
     gen = torch.Generator(device=gpu).manual_seed(1)
@@ -181,4 +180,4 @@ def test_fewer_rows_take_no_longer(gpu, fewer, more, heads, selected):
             end.record()
             torch.cuda.synchronize()
             best[i] = min(best[i], begin.elapsed_time(end))
-    assert best[0] < 1.06 * best[1], best
+    assert best[0] < 1.04 * best[1], best
